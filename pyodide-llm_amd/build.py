@@ -27,7 +27,7 @@ HIP_FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-ffp-contra
 ORDER = os.path.join(CSRC, "decode_order.txt")
 ORDER_FLAGS = ["-ffunction-sections", "-Xoffload-linker", f"--symbol-ordering-file={ORDER}", "-Xoffload-linker",
                "--no-warn-symbol-ordering"]
-SOURCES = ["gemv.hip", "gemm.hip", "misc.hip", "forms.hip", "attention.hip", "attention_tokens.hip", "sampling.hip",
+SOURCES = ["gemv.hip", "gemm.hip", "gemm_chains.hip", "misc.hip", "forms.hip", "attention.hip", "attention_tokens.hip", "sampling.hip",
            "ceilings.hip", "engine.cpp"]
 
 

@@ -282,4 +282,23 @@ __device__ __forceinline__ void quantize_group(float v, int8_t *xq, float *xs, i
   if ((threadIdx.x & 31) == 0) xs[g] = scale;
 }
 
+// quantize_x of one group of 32 held four values a lane by its 8 lanes (aligned, all present): the largest magnitude
+// by the lanes' own maxima and three DPP steps (xor 1, xor 2, the mirror across the two quads), the scale and its
+// reciprocal as quantize_group computes them, four bytes stored at xq[j..j+3]
+__device__ __forceinline__ void quantize_group4(float4 o, int8_t *xq, float *xs, int j, int g, int32_t bias) {
+  float a = __builtin_fmaxf(__builtin_fmaxf(__builtin_fabsf(o.x), __builtin_fabsf(o.y)),
+                            __builtin_fmaxf(__builtin_fabsf(o.z), __builtin_fabsf(o.w)));
+  a = __builtin_fmaxf(a, __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(a), 0xB1, 0xF, 0xF, true)));
+  a = __builtin_fmaxf(a, __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(a), 0x4E, 0xF, 0xF, true)));
+  a = __builtin_fmaxf(a, __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(a), 0x141, 0xF, 0xF, true)));
+  const float qmax = bias == 0 ? 127.0f : 63.0f;
+  const float scale = a / qmax;
+  const float inv = scale > 0 ? 1.0f / scale : 0.0f;
+  const uint32_t q = (uint32_t)(uint8_t)quant_value(o.x, inv, bias) | ((uint32_t)(uint8_t)quant_value(o.y, inv, bias) << 8) |
+                     ((uint32_t)(uint8_t)quant_value(o.z, inv, bias) << 16) |
+                     ((uint32_t)(uint8_t)quant_value(o.w, inv, bias) << 24);
+  *reinterpret_cast<uint32_t *>(xq + j) = q;
+  if ((threadIdx.x & 7) == 0) xs[g] = scale;
+}
+
 }  // namespace ple

@@ -28,6 +28,13 @@ namespace {
 
 thread_local std::string g_error;
 
+// whether m tokens against rows of k go to the GEMM: more than the GEMV takes (rows that it does not take at all: more
+// than 8 tokens of bias 64, the rest is refused)
+bool on_gemm(int32_t k, int32_t m, bool relaxed) {
+  const int32_t most = gemv_tokens(k, relaxed);
+  return most < 1 ? relaxed && m > 8 : m > most;
+}
+
 int32_t fail(int32_t code, const std::string &what) {
   g_error = what;
   return code;
@@ -440,7 +447,7 @@ int32_t open_common(const he_config *cfg, const he_tensor *tensors, uint64_t siz
   // the tokens of one pass through the layers: a prompt block up to 1024 (the attention runs them in pieces of
   // ATTN_ROWS; measured at the 8B shape: 512 a pass 19.5k prompt tok/s, 1024 19.6k, 2048 18.5k; with the two-tile
   // GEMM 1024 20.5k, 2048 0.3% more for twice the activations)
-  e->chunk = std::min(max_block, e->c.relaxed ? 1024 : 16);
+  e->chunk = std::min(max_block, 1024);
   HIP_TRY(hipStreamCreateWithFlags(&e->stream, hipStreamNonBlocking));
   if ((rc = plan_regions(e))) return rc;
   if ((rc = dev_alloc(&e->blob, e->blob_bytes))) return rc;
@@ -487,42 +494,30 @@ struct F32Source {
 hipError_t matmul_launch(he_engine *e, const MatSeg *segs, int nseg, int32_t k, int32_t m, const int8_t *xq,
                          const float *xs, const F32Source *f32 = nullptr, const QkvFuse *qkv = nullptr,
                          bool persistent = false) {
-  const int32_t xq_stride = e->widest, xs_stride = e->widest / 32;
-  const int32_t step = gemv_tokens(k, e->c.relaxed);
-  if (step < 1) return hipErrorInvalidValue;
-  for (int32_t t0 = 0; t0 < m; t0 += step) {
-    MatArgs a{};
-    a.nseg = nseg;
-    a.total_rows = 0;
-    for (int i = 0; i < nseg; ++i) {
-      a.seg[i] = segs[i];
-      a.seg[i].y = segs[i].y + (int64_t)t0 * segs[i].y_stride;
-      a.total_rows += segs[i].rows;
-    }
-    a.xq = xq + (int64_t)t0 * xq_stride;
-    a.xs = xs + (int64_t)t0 * xs_stride;
-    a.xq_stride = xq_stride;
-    a.xs_stride = xs_stride;
-    a.k = k;
-    a.m = std::min(step, m - t0);
-    a.sums = nullptr;
-    if (f32) {
-      a.xf = f32->x;
-      a.xnorm = f32->norm;
-      a.eps = e->c.rms_norm_eps;
-    }
-    if (qkv) a.qkv = *qkv;
-    a.persistent = persistent && a.m == 1 && decode_persistent(k, e->c.six != 0, e->c.relaxed != 0);
-    hipError_t err = launch_gemv(a, e->c.six, e->c.relaxed, e->stream);
-    if (err != hipSuccess) return err;
+  MatArgs a{};
+  a.nseg = nseg;
+  for (int i = 0; i < nseg; ++i) {
+    a.seg[i] = segs[i];
+    a.total_rows += segs[i].rows;
   }
-  return hipSuccess;
+  a.xq = xq;
+  a.xs = xs;
+  a.xq_stride = e->widest;
+  a.xs_stride = e->widest / 32;
+  a.k = k;
+  a.m = m;
+  if (f32) {
+    a.xf = f32->x;
+    a.xnorm = f32->norm;
+    a.eps = e->c.rms_norm_eps;
+  }
+  if (qkv) a.qkv = *qkv;
+  a.persistent = persistent && m == 1 && decode_persistent(k, e->c.six != 0, e->c.relaxed != 0);
+  return launch_gemv(a, e->c.six, e->c.relaxed, e->stream);
 }
 
 // more tokens than one GEMV launch takes go to the MFMA GEMM (the same bits per token and row)
-bool use_gemm(const he_engine *e, int32_t k, int32_t m) {
-  return m > GEMV_MOST && gemm_supported(k, e->c.relaxed != 0);
-}
+bool use_gemm(const he_engine *e, int32_t k, int32_t m) { return on_gemm(k, m, e->c.relaxed != 0); }
 
 hipError_t gemm_launch(he_engine *e, const MatSeg *segs, int nseg, int32_t k, int32_t m, const int8_t *xq,
                        const float *xs) {
@@ -557,7 +552,7 @@ hipError_t gemm_glu_launch(he_engine *e, const MatSeg *w13, int32_t k, int32_t m
   a.k = k;
   a.m = m;
   a.glu = GluOut{gq, gs, e->widest, e->widest / 32, e->bias};
-  return launch_gemm_glu(a, e->c.six, e->stream);
+  return launch_gemm_glu(a, e->c.six, e->c.relaxed, e->stream);
 }
 
 // whether a chunk of m tokens takes the GEMM's SwiGLU epilogue: the w1 / w3 matmul on the GEMM, hidden units in whole
@@ -1353,21 +1348,10 @@ int32_t hk_matmul(void *y, const void *xq, const void *xs, const void *w, const 
   if (rc) return rc;
   if (!y || !xs || !ws) return fail(HE_E_ARG, "matmul: a required pointer is null");
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  if (m > GEMV_MOST && gemm_supported(k, bias == 64)) {
-    base.m = m;
-    HIP_TRY(launch_gemm(base, six != 0, bias == 64, s));
-    return HE_OK;
-  }
-  const int32_t step = gemv_tokens(k, bias == 64);
-  if (step < 1) return fail(HE_E_ARG, "matmul: rows too long for the GEMV");
-  for (int32_t t0 = 0; t0 < m; t0 += step) {
-    MatArgs a = base;
-    a.m = std::min(step, m - t0);
-    a.xq = base.xq + (int64_t)t0 * k;
-    a.xs = base.xs + (int64_t)t0 * (k / 32);
-    a.seg[0].y = base.seg[0].y + (int64_t)t0 * rows;
-    HIP_TRY(launch_gemv(a, six != 0, bias == 64, s));
-  }
+  base.m = m;
+  const bool gemm = on_gemm(k, m, bias == 64);
+  if (!gemm && gemv_tokens(k, bias == 64) < 1) return fail(HE_E_ARG, "matmul: rows too long for the GEMV");
+  HIP_TRY(gemm ? launch_gemm(base, six != 0, bias == 64, s) : launch_gemv(base, six != 0, bias == 64, s));
   return HE_OK;
 }
 
@@ -1379,7 +1363,7 @@ int32_t hk_group_sums(void *s, const void *xq, const void *w, int32_t m, int32_t
   if (!s) return fail(HE_E_ARG, "sums is null");
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   if (gemm) {
-    if (!gemm_supported(k, bias == 64)) return fail(HE_E_ARG, "the MFMA GEMM takes bias 64 only");
+    if (bias != 64) return fail(HE_E_ARG, "the MFMA GEMM takes bias 64 only");
     base.m = m;
     base.sums = reinterpret_cast<int32_t *>(s);
     HIP_TRY(launch_gemm(base, six != 0, true, st));

@@ -1,5 +1,5 @@
-// gemm.hip — the prefill matmul on CDNA4 i8 MFMA: many tokens against an int8 (or int6) matrix with per-group
-// float32 scales, in the reference's exact float32 order (kernels/kernel_relaxed.ts:34-67 matmul_q8r and :164-183
+// gemm.hip — the prefill matmul on CDNA4 i8 MFMA (bias 64): many tokens against an int8 (or int6) matrix with per-group
+// float32 scales (grids that these blocks fill; gemm_chains.hip takes the others, and bias 0), in the reference's exact float32 order (kernels/kernel_relaxed.ts:34-67 matmul_q8r and :164-183
 // matmul_q8r_tile, which is the same per (row, token); matmul_q6r :189-218 on the six.ts-widened values).
 //
 // For a (row r, token t): S_g = dot(w_g, q_g - 64) is an exact int32 per group g of 32. One
@@ -349,11 +349,10 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2))) void ge
 
 }  // namespace
 
-bool gemm_supported(int32_t k, bool relaxed) { return relaxed && k >= 32 && k % 32 == 0; }
-
 hipError_t launch_gemm(const MatArgs &a, bool six, bool relaxed, hipStream_t s) {
-  if (a.m < 1 || a.total_rows < 1 || !gemm_supported(a.k, relaxed)) return hipErrorInvalidValue;
-  if (a.sums && a.nseg != 1) return hipErrorInvalidValue;
+  if (a.m < 1 || a.total_rows < 1 || a.k < 32 || a.k % 32) return hipErrorInvalidValue;
+  if (a.sums && (a.nseg != 1 || !relaxed)) return hipErrorInvalidValue;
+  if (!a.sums && (!relaxed || gemm_chains_faster(a.total_rows, a.m, false))) return launch_gemm_chains(a, six, relaxed, s);
   const int64_t blocks = (int64_t)((a.total_rows + BR - 1) / BR) * ((a.m + BT - 1) / BT);
   if (blocks > (1ll << 30)) return hipErrorInvalidValue;
   const dim3 grid((unsigned)blocks);
@@ -371,15 +370,16 @@ hipError_t launch_gemm(const MatArgs &a, bool six, bool relaxed, hipStream_t s) 
   return hipGetLastError();
 }
 
-hipError_t launch_gemm_glu(const MatArgs &a, bool six, hipStream_t s) {
+hipError_t launch_gemm_glu(const MatArgs &a, bool six, bool relaxed, hipStream_t s) {
   const GluOut &g = a.glu;
-  if (a.m < 1 || a.nseg != 2 || a.sums || !gemm_supported(a.k, true)) return hipErrorInvalidValue;
+  if (a.m < 1 || a.nseg != 2 || a.sums || a.k < 32 || a.k % 32) return hipErrorInvalidValue;
   const int hidden = a.seg[0].rows;
   if (hidden < 32 || hidden % 32 || a.seg[1].rows != hidden || a.total_rows != 2 * hidden) return hipErrorInvalidValue;
   // the output's 4-byte runs and its scales: every store aligned and inside [m][q_stride] / [m][s_stride]
   if (!g.q || !g.s || (g.bias != 0 && g.bias != 64) || g.q_stride < hidden || g.q_stride % 4 ||
       g.s_stride < hidden / 32 || reinterpret_cast<uintptr_t>(g.q) % 4)
     return hipErrorInvalidValue;
+  if (!relaxed || gemm_chains_faster(a.total_rows, a.m, true)) return launch_gemm_chains_glu(a, six, relaxed, s);
   const int64_t blocks = (int64_t)(hidden / 32) * ((a.m + BT - 1) / BT);
   if (blocks > (1ll << 30)) return hipErrorInvalidValue;
   if (six)

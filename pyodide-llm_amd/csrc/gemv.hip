@@ -1,4 +1,4 @@
-// gemv.hip — the decode matmul (m <= 8 tokens) of int8/int6 rows against quantized activations, to the bit of the
+// gemv.hip — the decode matmul (one token; up to 6 with bias 0) of int8/int6 rows against quantized activations, to the bit of the
 // reference's CPU kernels:
 //   bias 64: kernels/kernel_relaxed.ts:34-67 matmul_q8r (and :195-218 matmul_q6r): per group the exact integer
 //            S_g = dot(w, q - 64); lane g % 4 of four float32 accumulators adds f32(S_g) * f32(ws * xs) for the groups
@@ -958,26 +958,32 @@ hipError_t launch_m(const MatArgs &a, hipStream_t s) {
 
 template <bool SIX, bool RELAXED, bool SUMS>
 hipError_t launch_sel(const MatArgs &a, hipStream_t s) {
-  switch (a.m) {
-    case 1: return launch_m<1, SIX, RELAXED, SUMS>(a, s);
-    case 2: return launch_m<2, SIX, RELAXED, SUMS>(a, s);
-    case 3: return launch_m<3, SIX, RELAXED, SUMS>(a, s);
-    case 4: return launch_m<4, SIX, RELAXED, SUMS>(a, s);
-    case 5: return launch_m<5, SIX, RELAXED, SUMS>(a, s);
-    case 6: return launch_m<6, SIX, RELAXED, SUMS>(a, s);
-    case 7: return launch_m<7, SIX, RELAXED, SUMS>(a, s);
-    case 8: return launch_m<8, SIX, RELAXED, SUMS>(a, s);
-    default: return hipErrorInvalidValue;
+  if (a.m == 1) return launch_m<1, SIX, RELAXED, SUMS>(a, s);
+  if constexpr (SUMS || !RELAXED) {
+    switch (a.m) {
+      case 2: return launch_m<2, SIX, RELAXED, SUMS>(a, s);
+      case 3: return launch_m<3, SIX, RELAXED, SUMS>(a, s);
+      case 4: return launch_m<4, SIX, RELAXED, SUMS>(a, s);
+      case 5: return launch_m<5, SIX, RELAXED, SUMS>(a, s);
+      case 6: return launch_m<6, SIX, RELAXED, SUMS>(a, s);
+    }
   }
+  if constexpr (SUMS) {
+    if (a.m == 7) return launch_m<7, SIX, RELAXED, SUMS>(a, s);
+    if (a.m == 8) return launch_m<8, SIX, RELAXED, SUMS>(a, s);
+  }
+  return hipErrorInvalidValue;
 }
 
 }  // namespace
 
 int32_t gemv_tokens(int32_t k, bool relaxed) {
-  // the most tokens one launch takes: 8, fewer where a block's products would pass 64 KiB of LDS
+  // none where a block's products of one token pass 64 KiB of LDS. Bias 64: one token (two go to the GEMM: 4096 x 4096
+  // 8.2 against 10.7 us here, 4096 x 14336 21.1 against 22.1). Bias 0: up to 6, fewer where their products pass the LDS
+  // (4096 x 4096, 6 tokens 15.6 against 17.0 us in the GEMM, 8 tokens 24.4 against 17.0).
   const size_t per_token = sizeof(float) * WAVES * (size_t)row_layout(k, relaxed).stride;
-  int32_t m = (int32_t)((64 * 1024) / per_token);
-  return m < 1 ? 0 : (m > 8 ? 8 : m);
+  const int32_t m = (int32_t)((64 * 1024) / per_token), most = relaxed ? 1 : 6;
+  return m > most ? most : m;
 }
 
 bool decode_takes_f32(int32_t k, bool six, bool relaxed) {

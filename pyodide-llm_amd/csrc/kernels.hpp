@@ -85,10 +85,8 @@ struct MatArgs {
 // the launch goes another way
 int32_t decode_block_rows(int32_t k, int32_t total_rows, bool six, bool relaxed, bool xf, bool qkv_on);
 
-// the most tokens the engine gives one GEMV pass: more go to the MFMA GEMM where it takes them
-constexpr int32_t GEMV_MOST = 8;
-
-// decode GEMV, m <= 8 tokens: exact int32 group sums, the reference's float32 order
+// decode GEMV: exact int32 group sums, the reference's float32 order; bias 64 one token, bias 0 up to 6 (m <=
+// gemv_tokens()), with a.sums up to 8
 hipError_t launch_gemv(const MatArgs &a, bool six, bool relaxed, hipStream_t s);
 // whether a one-token launch_gemv of rows of k takes its activations as float32 (MatArgs.xf)
 bool decode_takes_f32(int32_t k, bool six, bool relaxed);
@@ -96,14 +94,19 @@ bool decode_takes_f32(int32_t k, bool six, bool relaxed);
 bool decode_persistent(int32_t k, bool six, bool relaxed);
 // whether a one-token launch_gemv of rows of k finishes q / k / v itself (MatArgs.qkv)
 bool decode_fuses_qkv(int32_t k, bool six, bool relaxed);
-// the most tokens one launch_gemv takes for rows of k (its products of a row fit the block's LDS)
+// the most tokens one launch_gemv takes for rows of k, 0 where a row's products pass the block's LDS; more tokens go to
+// launch_gemm
 int32_t gemv_tokens(int32_t k, bool relaxed);
-// prefill GEMM on i8 MFMA, any m (bias 64, int8 or int6): the same bits as launch_gemv per (token, row); with
-// a.sums (one segment) the exact int32 group sums [m][rows][K/32] instead
+// GEMM on i8 MFMA, any m: the same bits as launch_gemv per (token, row); with a.sums (one segment, bias 64) the exact
+// int32 group sums [m][rows][K/32] instead
 hipError_t launch_gemm(const MatArgs &a, bool six, bool relaxed, hipStream_t s);
-// the w1 / w3 GEMM with the SwiGLU and its quantize_x in the epilogue (a.glu; bias 64 weights only)
-hipError_t launch_gemm_glu(const MatArgs &a, bool six, hipStream_t s);
-bool gemm_supported(int32_t k, bool relaxed);
+// the w1 / w3 GEMM with the SwiGLU and its quantize_x in the epilogue (a.glu)
+hipError_t launch_gemm_glu(const MatArgs &a, bool six, bool relaxed, hipStream_t s);
+// gemm_chains.hip: the GEMM with each float32 lane chain on a wave of its own, for bias 0 and for the grids where it is
+// the faster one (rows: of every segment). launch_gemm and launch_gemm_glu check the arguments and choose.
+bool gemm_chains_faster(int32_t rows, int32_t m, bool glu);
+hipError_t launch_gemm_chains(const MatArgs &a, bool six, bool relaxed, hipStream_t s);
+hipError_t launch_gemm_chains_glu(const MatArgs &a, bool six, bool relaxed, hipStream_t s);
 
 // quantize_x over m rows of n (x_stride apart) into xq (xq_stride) / xs (xs_stride)
 hipError_t launch_quantize(int8_t *xq, float *xs, const float *x, int32_t m, int32_t n, int32_t x_stride,

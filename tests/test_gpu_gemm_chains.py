@@ -1,0 +1,59 @@
+"""The matmuls of more tokens than the GEMV takes, to the bit of the oracle, at the edges of the GEMM's tiles and of the
+rules that pick one: 16 x 16, 32 x 32 and 64 x 32 blocks with a lane chain a wave, the 64 x 128 blocks of full grids, and
+the SwiGLU epilogue's 16, 32 and 48 tokens; both biases, int8 and int6, every number of groups past the fours."""
+import numpy as np
+import pytest
+
+import gpu_lib as gl
+import oracle_lib as ol
+from paths import package
+from test_gpu_kernels import activations, same_bits, weights
+
+pytestmark = pytest.mark.gpu
+
+# (rows, k, m): one row, one group; the last row and token of a tile and the first of the next; stages cut after each
+# number of groups
+SMALL = [(1, 32, 2), (16, 64, 15), (17, 288, 16), (33, 544, 17), (100, 480, 33)]
+MIDDLE = [(544, 352, 250), (513, 512, 241)]       # over 512 blocks of 16 x 16, at most 256 of 32 x 32
+LARGE = [(1090, 288, 260), (1100, 1120, 257)]     # over 256 blocks of 32 x 32
+FULL = [(2590, 96, 1170), (2560, 288, 1169)]      # the 64 x 128 blocks (bias 64)
+
+
+@pytest.mark.parametrize("bias", [64, 0])
+@pytest.mark.parametrize("six", [0, 1])
+@pytest.mark.parametrize("rows,k,m", SMALL + MIDDLE + LARGE + FULL)
+def test_matmul_bits(rows, k, m, six, bias):
+    w, ws = weights(rows, k, six)
+    xq, xs = activations(m, k, bias)
+    assert same_bits(gl.matmul(xq, xs, w, ws, rows, k, bias, six), ol.matmul(xq, xs, w, ws, rows, k, bias, six))
+
+
+@pytest.mark.parametrize("m", [2, 6, 7, 8, 9])
+def test_where_the_gemv_ends(m):
+    """bias 0: up to 6 tokens on the GEMV (2 where a row's products are long), more on the GEMM"""
+    for k in (96, 14336):
+        w, ws = weights(40, k, 0)
+        xq, xs = activations(m, k, 0)
+        assert same_bits(gl.matmul(xq, xs, w, ws, 40, k, 0, 0), ol.matmul(xq, xs, w, ws, 40, k, 0, 0)), k
+
+
+@pytest.mark.parametrize("relaxed", [1, 0])
+@pytest.mark.parametrize("six", [0, 1])
+@pytest.mark.parametrize("hidden,m", [(96, 5), (2784, 16), (2784, 40), (2784, 97)])
+def test_swiglu_epilogue_bits(hidden, m, six, relaxed):
+    """a prompt block whose w1 / w3 GEMM finishes the SwiGLU: the second layer's keys and values follow from every token's
+    output of the first layer's"""
+    cfg = ol.config(dim=288, hidden_dim=hidden, n_layers=2, n_heads=6, n_kv_heads=6, head_size=48, vocab_size=320,
+                    seq_len=128, shared_classifier=0, six=six, relaxed=relaxed)
+    tensors, size = ol.places(cfg)
+    ck = ol.vary_vectors(cfg, tensors, ol.synth_checkpoint(cfg, tensors, size, seed=4), seed=5)
+    cos, sin = ol.rope_tables(cfg.seq_len, cfg.head_size, 10000.0)
+    tokens = [int(t) for t in np.random.default_rng(m).integers(0, cfg.vocab_size, size=m)]
+    ref = ol.Model(cfg, tensors, ck, cos, sin, max_block=128)
+    eng = package().open_config(cfg, tensors, ck, cos, sin, max_block=128)
+    ref.run(tokens, 0, False)
+    eng.forwardMany(tokens, 0)
+    kv, (k, v) = eng.keysAndValues(0, m), ref.kv(0, m)
+    assert same_bits(kv["keys"], k.reshape(-1)) and same_bits(kv["values"], v.reshape(-1))
+    eng.release()
+    ref.close()
