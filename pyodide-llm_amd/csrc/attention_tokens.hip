@@ -23,6 +23,21 @@ namespace {
 // add a product instead of a multiply and an add. The head is staged in chunks of DC dims (the rows' queries and the
 // tile's keys, double buffered in LDS: the next chunk's loads in flight while this one is summed). No tile maxima:
 // the softmax takes each row's largest score from the scores themselves.
+// The blocks of the prompt's kernels by XCD: block b runs on XCD b % 8, and the (kv head, token block, x) triples, x
+// fastest, are dealt to the XCDs in 8 contiguous ranges, so that what the blocks of a kv head share (its keys and
+// values, the score rows that one kernel writes and the next reads) stays in one XCD's L2. A kv head's token blocks come
+// from both ends in turn: the later ones see more positions, and where a kv head's blocks are cut between two XCDs both
+// get short and long ones.
+struct TokenBlock {
+  int x, kh, z;
+};
+__device__ __forceinline__ TokenBlock token_block(int nx, int nz) {
+  const int n = gridDim.x, xcd = blockIdx.x & 7;
+  const int idx = xcd * (n / 8) + min(xcd, n % 8) + (blockIdx.x >> 3);
+  const int rest = idx / nx, zi = rest % nz;
+  return {idx % nx, rest / nz, (zi & 1) ? nz - 1 - zi / 2 : zi / 2};
+}
+
 template <int HS> constexpr int score_chunk() { return HS % 32 == 0 ? 32 : 16; }
 constexpr int SCORE_ROWS = 64;  // (token, head) rows a block
 
@@ -397,6 +412,92 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void p
   }
 }
 
+// (C') for grids too small to fill the chip with (C)'s one wave a tile: four waves share one tile of 16 (token, head) rows
+// x 16 columns. A wave takes every fourth run of 16 positions (four whole fours): lane (g, i) reads four g of the run of
+// row i's weights and of column i's values straight from memory (no staging: no other wave reads them), and four MFMAs,
+// element e of block g being position 4g + e, leave it the products of each four of its 4 outputs, added
+// (p0 v0 + p1 v1) + (p2 v2 + p3 v3). The sums of a round (64 positions, 16 fours) meet in LDS, and each thread adds
+// one of the 256 outputs in order, one add a four: the serial chain is that add alone, where (C)'s wave also makes
+// every product and sum of its tile between two of them.
+constexpr int PR = 64;  // positions a round
+template <int HS, bool HALF>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void pv4_tokens_kernel(const AttnArgs a) {
+  __shared__ float4 sums[2][PR / 4][64];  // [buffer][four][lane]: the lane's 4 outputs
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 4, l16 = lane & 15;
+  const int mul = a.nh / a.nkv, tt_n = max(1, 16 / mul);
+  const TokenBlock tb = token_block(HS / 16, (a.m + tt_n - 1) / tt_n);
+  const int kh = tb.kh, j0 = tb.x * 16, t0 = tb.z * tt_n, last = min(t0 + tt_n, a.m) - 1;
+  const int pos0 = first_position(a);
+  const int most4 = (pos0 + last + 1) & ~3;  // the block's last token's whole fours: every four any row adds
+  const int least4 = (pos0 + t0 + 1) & ~3;   // the first token's: every row adds the fours below it
+  const int rounds = (most4 + PR - 1) / PR;
+  // the weights of row l16 (token clamped to the block's last) and the values of column l16
+  const float *prow = a.scores + ((int64_t)min(t0 + l16 / mul, last) * a.nh + kh * mul + l16 % mul) * a.seq_len;
+  const int64_t vrow = (int64_t)(kh * HS + j0 + l16) * a.vstride;
+  // this thread's output: register tid % 4 of lane tid / 4, that is row 4 (lane / 16) + register, column lane % 16 (the
+  // 64 lanes of a wave read 64 floats side by side); its whole fours
+  const int r = 4 * (tid >> 6) + (tid & 3), tt = r / mul, t = t0 + tt;
+  const int count = pos0 + min(t, last) + 1, nb = (count & ~3) >> 2;
+  float acc = 0.0f;
+  constexpr int D = 2;  // rounds of loads in flight
+  float4 pf[D], vf[D];
+  auto fetch = [&](int round, float4 &p4, float4 &v4) {
+    const int po = max(min(round * PR + wave * 16 + 4 * g, most4 - 4), 0);  // clamped: loaded, never added
+    p4 = *reinterpret_cast<const float4 *>(prow + po);
+    v4 = cache4<HALF>(a.vcache, vrow + po);
+  };
+  const v16f zero = {};
+  auto step = [&](int round, float4 &p4, float4 &v4) {
+    const v16f d0 = __builtin_amdgcn_mfma_f32_16x16x1f32(p4.x, v4.x, zero, 0, 0, 0);
+    const v16f d1 = __builtin_amdgcn_mfma_f32_16x16x1f32(p4.y, v4.y, zero, 0, 0, 0);
+    const v16f d2 = __builtin_amdgcn_mfma_f32_16x16x1f32(p4.z, v4.z, zero, 0, 0, 0);
+    const v16f d3 = __builtin_amdgcn_mfma_f32_16x16x1f32(p4.w, v4.w, zero, 0, 0, 0);
+    fetch(round + D, p4, v4);
+    float4(*const out)[64] = sums[round & 1];
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+      float o[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) o[q] = (d0[4 * b + q] + d1[4 * b + q]) + (d2[4 * b + q] + d3[4 * b + q]);
+      out[wave * 4 + b][lane] = make_float4(o[0], o[1], o[2], o[3]);
+    }
+    lds_barrier();  // (the other buffer's last readers passed the one before)
+    const float *in = reinterpret_cast<const float *>(out) + tid;
+    float x[PR / 4];
+#pragma unroll
+    for (int b = 0; b < PR / 4; ++b) x[b] = in[b * 256];
+    pin16(x);  // (read whole, with one wait: a read under each four's test would be waited for by itself)
+    if ((round + 1) * PR <= least4) {  // uniform: every row of the block adds every four of the round
+#pragma unroll
+      for (int b = 0; b < PR / 4; ++b) acc = acc + x[b];
+    } else {
+      const int left = nb - round * (PR / 4);
+#pragma unroll
+      for (int b = 0; b < PR / 4; ++b) {
+        const float next = acc + x[b];
+        acc = b < left ? next : acc;
+      }
+    }
+  };
+#pragma unroll
+  for (int d = 0; d < D; ++d) fetch(d, pf[d], vf[d]);
+  int c = 0;
+  for (; c + D <= rounds; c += D) {
+#pragma unroll
+    for (int d = 0; d < D; ++d) step(c + d, pf[d], vf[d]);
+  }
+#pragma unroll
+  for (int d = 0; d < D - 1; ++d)
+    if (c + d < rounds) step(c + d, pf[d], vf[d]);  // uniform
+  // the positions past the row's fours, one at a time
+  if (tt >= tt_n || t >= a.m) return;
+  const int hh = kh * mul + r % mul, col = j0 + ((tid >> 2) & 15);
+  const float *pt = a.scores + ((int64_t)t * a.nh + hh) * a.seq_len;
+  const int64_t vcol = (int64_t)(kh * HS + col) * a.vstride;
+  for (int p = count & ~3; p < count; ++p) acc = acc + pt[p] * cache1<HALF>(a.vcache, vcol + p);
+  a.out[(int64_t)t * a.out_stride + hh * HS + col] = acc;
+}
+
 template <int HS, bool HALF>
 hipError_t scores_tokens_hs(const AttnArgs &a, hipStream_t s) {
   // the kernel's element offsets are 32-bit
@@ -437,6 +538,14 @@ hipError_t softmax_pv_hs(const AttnArgs &a, hipStream_t s) {
   }
   constexpr int C = pv_cols<HS>();
   const int tt = std::max(1, (1024 / C) / (a.nh / a.nkv));  // tokens a block
+  // up to one and a half of (C)'s blocks a CU: four waves a tile (a pass of 37 tokens at position 1500, 32 / 8 heads of
+  // 128, 160 blocks: 43.9 -> 24.0 us; 512 tokens, 8 heads of 64, 256: 22.0 -> 11.7; a 512-token prompt of 12 heads of 64
+  // at position 400, 384: 5% of the whole; 129 tokens of the first shape, 544: 0.4% slower; 2048: 99 -> 146 us)
+  if (HS / C * a.nkv * ((a.m + tt - 1) / tt) <= 384) {
+    const int t4 = std::max(1, 16 / (a.nh / a.nkv));
+    hipLaunchKernelGGL((pv4_tokens_kernel<HS, HALF>), dim3(HS / 16 * a.nkv * ((a.m + t4 - 1) / t4)), dim3(256), 0, s, a);
+    return hipGetLastError();
+  }
   hipLaunchKernelGGL((pv_tokens_kernel<HS, HALF>), dim3(HS / C, a.nkv, (a.m + tt - 1) / tt), dim3(256), 0, s, a);
   return hipGetLastError();
 }
