@@ -511,16 +511,7 @@ int32_t attention_most_positions() {
 }
 
 bool attention_quantizes(const AttnArgs &a) {
-  if (!attention_supported(a.hs, a.nh, a.nkv) || a.m > DECODE_TOKENS || a.hs % 32 || a.split) return false;
-  int nslot = 0;
-  switch (a.hs) {
-    case 32: return attend_lds<32>(a, &nslot) > 0;
-    case 64: return attend_lds<64>(a, &nslot) > 0;
-    case 96: return attend_lds<96>(a, &nslot) > 0;
-    case 128: return attend_lds<128>(a, &nslot) > 0;
-    case 256: return attend_lds<256>(a, &nslot) > 0;
-    default: return false;
-  }
+  return attention_supported(a.hs, a.nh, a.nkv) && a.hs % 32 == 0;
 }
 
 hipError_t launch_attention(const AttnArgs &a, hipStream_t s) {

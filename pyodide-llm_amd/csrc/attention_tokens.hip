@@ -286,6 +286,18 @@ __global__ __launch_bounds__(256) void softmax4_kernel(const AttnArgs a) {
   }
 }
 
+// quantize_x of 32 columns (j0 .. of kv head kh's query heads: one group) of R (token, head) rows in LDS, 8 lanes a row:
+// into a.xq / a.xs. The whole block calls it (8 R threads or more).
+template <int HS, int R>
+__device__ __forceinline__ void quantize_rows(const AttnArgs &a, const float *rows, int stride, int kh, int j0, int t0,
+                                              int tt_n, int mul, int tid) {
+  const int r = tid >> 3, tt = r / mul, t = t0 + tt;
+  if (r >= R || tt >= tt_n || t >= a.m) return;  // (a row's 8 lanes leave together)
+  const int at = (kh * mul + r % mul) * HS + j0;
+  quantize_group4(*reinterpret_cast<const float4 *>(rows + r * stride + 4 * (tid & 7)),
+                  a.xq + (int64_t)t * a.xq_stride, a.xs + (int64_t)t * a.xs_stride, at + 4 * (tid & 7), at / 32, a.bias);
+}
+
 // (C) for many tokens (a prompt block), products on the matrix core: v_mfma_f32_16x16x1_4b_f32 with a zero
 // accumulator makes 4 x 16 x 16 single products, block b of the four being position 4k + b: p[row][4k + b] *
 // v[4k + b][col], each the correctly rounded float32 product. A lane then holds, for each of its 4 (row, column)
@@ -397,9 +409,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void p
   }
 #undef PV_FETCH
 #undef PV_STAGE
-  // each row's positions past its fours, one at a time, then the outputs
+  // each row's positions past its fours, one at a time, then the outputs; with a.xq through LDS to quantize_x of the
+  // block's 32 columns, a group of each row
   const int col = j0 + tcol + l16;
   const int64_t vcol = (int64_t)(kh * HS + col) * a.vstride;
+  const bool quantized = C == 32 && a.xq;  // uniform
+  float *const rows = ps[0];               // [R][C + 4] (ps holds 2 R (TPC + 4) floats)
+  if (quantized) __syncthreads();          // the last chunk's readers
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
     const int r = trow + g * 4 + q, tt = r / mul, t = t0 + tt;
@@ -408,7 +424,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void p
     const float *pt = a.scores + ((int64_t)t * a.nh + hh) * a.seq_len;
     float o = acc[q];
     for (int p = count & ~3; p < count; ++p) o = o + pt[p] * cache1<HALF>(a.vcache, vcol + p);
-    a.out[(int64_t)t * a.out_stride + hh * HS + col] = o;
+    if (quantized) rows[r * (C + 4) + tcol + l16] = o;
+    else a.out[(int64_t)t * a.out_stride + hh * HS + col] = o;
+  }
+  if (quantized) {
+    __syncthreads();
+    quantize_rows<HS, R>(a, rows, C + 4, kh, j0, t0, tt_n, mul, tid);
   }
 }
 
@@ -419,21 +440,26 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void p
 // (p0 v0 + p1 v1) + (p2 v2 + p3 v3). The sums of a round (64 positions, 16 fours) meet in LDS, and each thread adds
 // one of the 256 outputs in order, one add a four: the serial chain is that add alone, where (C)'s wave also makes
 // every product and sum of its tile between two of them.
+// A block is one tile, or two side by side (32 columns: a quantization group, finished by quantize_x where a.xq asks).
 constexpr int PR = 64;  // positions a round
+template <int HS> constexpr int pv4_tiles() { return HS % 32 == 0 ? 2 : 1; }
 template <int HS, bool HALF>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void pv4_tokens_kernel(const AttnArgs a) {
-  __shared__ float4 sums[2][PR / 4][64];  // [buffer][four][lane]: the lane's 4 outputs
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 4, l16 = lane & 15;
+__global__ __launch_bounds__(256 * pv4_tiles<HS>()) __attribute__((amdgpu_waves_per_eu(2))) void pv4_tokens_kernel(
+    const AttnArgs a) {
+  constexpr int NC = pv4_tiles<HS>();
+  __shared__ float4 sums[NC][2][PR / 4][64];  // [tile][buffer][four][lane]: the lane's 4 outputs
+  const int tile = NC == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+  const int tid = threadIdx.x & 255, lane = tid & 63, wave = tid >> 6, g = lane >> 4, l16 = lane & 15;
   const int mul = a.nh / a.nkv, tt_n = max(1, 16 / mul);
-  const TokenBlock tb = token_block(HS / 16, (a.m + tt_n - 1) / tt_n);
-  const int kh = tb.kh, j0 = tb.x * 16, t0 = tb.z * tt_n, last = min(t0 + tt_n, a.m) - 1;
+  const TokenBlock tb = token_block(HS / 16 / NC, (a.m + tt_n - 1) / tt_n);
+  const int kh = tb.kh, j0 = tb.x * 16 * NC, jt = j0 + tile * 16, t0 = tb.z * tt_n, last = min(t0 + tt_n, a.m) - 1;
   const int pos0 = first_position(a);
   const int most4 = (pos0 + last + 1) & ~3;  // the block's last token's whole fours: every four any row adds
   const int least4 = (pos0 + t0 + 1) & ~3;   // the first token's: every row adds the fours below it
   const int rounds = (most4 + PR - 1) / PR;
   // the weights of row l16 (token clamped to the block's last) and the values of column l16
   const float *prow = a.scores + ((int64_t)min(t0 + l16 / mul, last) * a.nh + kh * mul + l16 % mul) * a.seq_len;
-  const int64_t vrow = (int64_t)(kh * HS + j0 + l16) * a.vstride;
+  const int64_t vrow = (int64_t)(kh * HS + jt + l16) * a.vstride;
   // this thread's output: register tid % 4 of lane tid / 4, that is row 4 (lane / 16) + register, column lane % 16 (the
   // 64 lanes of a wave read 64 floats side by side); its whole fours
   const int r = 4 * (tid >> 6) + (tid & 3), tt = r / mul, t = t0 + tt;
@@ -453,7 +479,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void p
     const v16f d2 = __builtin_amdgcn_mfma_f32_16x16x1f32(p4.z, v4.z, zero, 0, 0, 0);
     const v16f d3 = __builtin_amdgcn_mfma_f32_16x16x1f32(p4.w, v4.w, zero, 0, 0, 0);
     fetch(round + D, p4, v4);
-    float4(*const out)[64] = sums[round & 1];
+    float4(*const out)[64] = sums[tile][round & 1];
 #pragma unroll
     for (int b = 0; b < 4; ++b) {
       float o[4];
@@ -490,12 +516,22 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void p
   for (int d = 0; d < D - 1; ++d)
     if (c + d < rounds) step(c + d, pf[d], vf[d]);  // uniform
   // the positions past the row's fours, one at a time
-  if (tt >= tt_n || t >= a.m) return;
-  const int hh = kh * mul + r % mul, col = j0 + ((tid >> 2) & 15);
-  const float *pt = a.scores + ((int64_t)t * a.nh + hh) * a.seq_len;
-  const int64_t vcol = (int64_t)(kh * HS + col) * a.vstride;
-  for (int p = count & ~3; p < count; ++p) acc = acc + pt[p] * cache1<HALF>(a.vcache, vcol + p);
-  a.out[(int64_t)t * a.out_stride + hh * HS + col] = acc;
+  const int hh = kh * mul + r % mul, col = jt + ((tid >> 2) & 15);
+  const bool live = tt < tt_n && t < a.m;
+  if (live) {
+    const float *pt = a.scores + ((int64_t)t * a.nh + hh) * a.seq_len;
+    const int64_t vcol = (int64_t)(kh * HS + col) * a.vstride;
+    for (int p = count & ~3; p < count; ++p) acc = acc + pt[p] * cache1<HALF>(a.vcache, vcol + p);
+  }
+  if (NC == 2 && a.xq) {  // uniform
+    float *const rows = reinterpret_cast<float *>(sums);  // [16][36]
+    __syncthreads();
+    if (live) rows[r * 36 + col - j0] = acc;
+    __syncthreads();
+    quantize_rows<HS, 16>(a, rows, 36, kh, j0, t0, tt_n, mul, threadIdx.x);
+  } else if (live) {
+    a.out[(int64_t)t * a.out_stride + hh * HS + col] = acc;
+  }
 }
 
 template <int HS, bool HALF>
@@ -543,7 +579,8 @@ hipError_t softmax_pv_hs(const AttnArgs &a, hipStream_t s) {
   // at position 400, 384: 5% of the whole; 129 tokens of the first shape, 544: 0.4% slower; 2048: 99 -> 146 us)
   if (HS / C * a.nkv * ((a.m + tt - 1) / tt) <= 384) {
     const int t4 = std::max(1, 16 / (a.nh / a.nkv));
-    hipLaunchKernelGGL((pv4_tokens_kernel<HS, HALF>), dim3(HS / 16 * a.nkv * ((a.m + t4 - 1) / t4)), dim3(256), 0, s, a);
+    hipLaunchKernelGGL((pv4_tokens_kernel<HS, HALF>), dim3(HS / 16 / pv4_tiles<HS>() * a.nkv * ((a.m + t4 - 1) / t4)),
+                       dim3(256 * pv4_tiles<HS>()), 0, s, a);
     return hipGetLastError();
   }
   hipLaunchKernelGGL((pv_tokens_kernel<HS, HALF>), dim3(HS / C, a.nkv, (a.m + tt - 1) / tt), dim3(256), 0, s, a);

@@ -520,7 +520,7 @@ hipError_t matmul_launch(he_engine *e, const MatSeg *segs, int nseg, int32_t k, 
 bool use_gemm(const he_engine *e, int32_t k, int32_t m) { return on_gemm(k, m, e->c.relaxed != 0); }
 
 hipError_t gemm_launch(he_engine *e, const MatSeg *segs, int nseg, int32_t k, int32_t m, const int8_t *xq,
-                       const float *xs) {
+                       const float *xs, const QkvFuse *qkv) {
   MatArgs a{};
   a.nseg = nseg;
   for (int i = 0; i < nseg; ++i) {
@@ -533,18 +533,20 @@ hipError_t gemm_launch(he_engine *e, const MatSeg *segs, int nseg, int32_t k, in
   a.xs_stride = e->widest / 32;
   a.k = k;
   a.m = m;
+  if (qkv) a.qkv = *qkv;
   return launch_gemm(a, e->c.six, e->c.relaxed, e->stream);
 }
 
-// the prompt's w1 / w3 GEMM with the SwiGLU in its epilogue, writing quantize_x of its output to gq / gs
-// ([m][widest] bytes, [m][widest / 32] scales)
-hipError_t gemm_glu_launch(he_engine *e, const MatSeg *w13, int32_t k, int32_t m, const int8_t *xq, const float *xs,
-                           int8_t *gq, float *gs) {
+// the prompt's w1 / w3 GEMM with the SwiGLU in its epilogue (two segments), or w1's with the GELU (one, with its bias),
+// writing quantize_x of its output to gq / gs ([m][widest] bytes, [m][widest / 32] scales)
+hipError_t gemm_ffn_launch(he_engine *e, const MatSeg *segs, int nseg, int32_t k, int32_t m, const int8_t *xq,
+                           const float *xs, int8_t *gq, float *gs) {
   MatArgs a{};
-  a.nseg = 2;
-  a.seg[0] = w13[0];
-  a.seg[1] = w13[1];
-  a.total_rows = w13[0].rows + w13[1].rows;
+  a.nseg = nseg;
+  for (int i = 0; i < nseg; ++i) {
+    a.seg[i] = segs[i];
+    a.total_rows += segs[i].rows;
+  }
   a.xq = xq;
   a.xs = xs;
   a.xq_stride = e->widest;
@@ -552,14 +554,16 @@ hipError_t gemm_glu_launch(he_engine *e, const MatSeg *w13, int32_t k, int32_t m
   a.k = k;
   a.m = m;
   a.glu = GluOut{gq, gs, e->widest, e->widest / 32, e->bias};
-  return launch_gemm_glu(a, e->c.six, e->c.relaxed, e->stream);
+  return nseg == 2 ? launch_gemm_glu(a, e->c.six, e->c.relaxed, e->stream)
+                   : launch_gemm_gelu(a, e->c.six, e->c.relaxed, e->stream);
 }
 
-// whether a chunk of m tokens takes the GEMM's SwiGLU epilogue: the w1 / w3 matmul on the GEMM, hidden units in whole
-// groups, and the float32 buffers of h1 / h3 large enough for the quantized output ([chunk][widest] bytes in hb,
-// [chunk][widest / 32] floats in hb2)
-bool glu_in_gemm(const he_engine *e, int32_t m) {
+// whether a chunk of m tokens takes the GEMM's SwiGLU or GELU epilogue: the matmul on the GEMM (the GELU: on the one that
+// finishes it), hidden units in whole groups, and the float32 buffers of h1 / h3 large enough for the quantized output
+// ([chunk][widest] bytes in hb, [chunk][widest / 32] floats in hb2)
+bool ffn_in_gemm(const he_engine *e, int32_t m) {
   const int32_t hidden = e->c.hidden_dim;
+  if (layer_norm(e->c) && !gemm_finishes(hidden, m, e->c.relaxed != 0)) return false;
   return use_gemm(e, e->c.dim, m) && hidden % 32 == 0 && e->widest % 4 == 0 && e->widest <= 4 * (int64_t)hidden;
 }
 
@@ -567,7 +571,7 @@ hipError_t matmul(he_engine *e, const MatSeg *segs, int nseg, int32_t k, int32_t
                   const F32Source *f32 = nullptr, const QkvFuse *qkv = nullptr, bool persistent = false) {
   if (use_gemm(e, k, m))
     return timed(e, HE_K_GEMM, matmul_bytes(e, segs, nseg, k, m),
-                 [&] { return gemm_launch(e, segs, nseg, k, m, xq, xs); });
+                 [&] { return gemm_launch(e, segs, nseg, k, m, xq, xs, qkv); });
   return timed(e, HE_K_GEMV, matmul_bytes(e, segs, nseg, k, m),
                [&] { return matmul_launch(e, segs, nseg, k, m, xq, xs, f32, qkv, persistent); });
 }
@@ -663,8 +667,10 @@ int32_t run_chunk(he_engine *e, const int32_t *tokens, int32_t m, int32_t pos0, 
                                       m, dim, dim, W, W / 32, 0, e->bias, s);
       }));
     }
-    const bool fuse_qkv = c.arch == HE_ARCH_LLAMA && !c.qk_norm && m == 1 &&
-                          decode_fuses_qkv(dim, c.six != 0, c.relaxed != 0);
+    // the q/k/v matmul adds the biases, rotates q and k and writes k and v into the cache itself where it can (Qwen3's
+    // head norms stand between them)
+    const bool fuse_qkv = !c.qk_norm && (use_gemm(e, dim, m) ? gemm_finishes(qdim + 2 * kvdim, m, c.relaxed != 0)
+                                                             : m == 1 && decode_fuses_qkv(dim, c.six != 0, c.relaxed != 0));
     // one token of a small model (dim <= 1024): the q/k/v and w1/w3 GEMVs take the float32 token and run rmsnorm and
     // quantize_x in each block (an ordered sum of 256 steps at most), two launches a layer fewer. (At dim 4096 each
     // block repeating the 1024-step sum costs more than the launch.)
@@ -678,9 +684,8 @@ int32_t run_chunk(he_engine *e, const int32_t *tokens, int32_t m, int32_t pos0, 
       }));
     }
     if (fuse_qkv) {
-      // one token: the q/k/v GEMV adds the biases, rotates q and k and writes k and v into the cache itself
       const QkvFuse fuse{1, qp.bq, qp.bk, qp.bv, e->cos_t, e->sin_t, qp.kcache, qp.vcache, pos0, hs, kvdim, c.half_kv,
-                         qp.vstride, dpos};
+                         qp.vstride, dpos, qp.rot};
       HIP_TRY(matmul(e, qkv, 3, dim, m, e->xq, e->xs, norm_in_gemv ? &att_src : nullptr, &fuse));
     } else {
       HIP_TRY(matmul(e, qkv, 3, dim, m, e->xq, e->xs, norm_in_gemv ? &att_src : nullptr));
@@ -728,7 +733,14 @@ int32_t run_chunk(he_engine *e, const int32_t *tokens, int32_t m, int32_t pos0, 
     if (!quantized) at.xq = nullptr;
     double kv_rows = 0;
     for (int32_t t = 0; t < m; ++t) kv_rows += pos0 + t + 1;
-    const MatSeg wo[1] = {{e->mat(HE_T_WO, l), e->mat_scales(HE_T_WO, l), e->x, dim, dim, 1}};
+    // (GPT-2 and GPT-NeoX: x += wo(xb), then x += bo; w2 and b2 the same)
+    const MatSeg wo[1] = {{e->mat(HE_T_WO, l), e->mat_scales(HE_T_WO, l), e->x, dim, dim, 1,
+                           ln ? e->vec(HE_T_BO, (int64_t)l * dim) : nullptr}};
+    const MatSeg w2[1] = {{e->mat(HE_T_W2, l), e->mat_scales(HE_T_W2, l), e->x, dim, dim, 1,
+                           ln ? e->vec(HE_T_B2, (int64_t)l * dim) : nullptr}};
+    // where the GEMM finishes the FFN's activation and its quantize_x, its bytes and scales go where h1 and h3 would (hb
+    // and hb2 hold [chunk][W] bytes and [chunk][W / 32] floats: ffn_in_gemm checks), apart from its input in xq / xs
+    int8_t *const gq = reinterpret_cast<int8_t *>(e->hb);
     HIP_TRY(timed(e, HE_K_ATTENTION, kv_rows * 2 * kvdim * esz + (double)m * qdim * 8,
                   [&] { return launch_attention(at, s); }));
     if (quantized) {
@@ -743,24 +755,26 @@ int32_t run_chunk(he_engine *e, const int32_t *tokens, int32_t m, int32_t pos0, 
       HIP_TRY(matmul(e, wo, 1, qdim, m, e->xq, e->xs));
     }
     if (ln) {
-      // x += bo; LayerNorm of x (or of the layer's input: parallel residual); w1; gelu(+ b1); w2; x += b2
-      HIP_TRY(timed(e, HE_K_ELEMENTWISE, (double)m * dim * 12,
-                    [&] { return launch_add_rows(e->x, e->vec(HE_T_BO, (int64_t)l * dim), m, dim, dim, s); }));
+      // LayerNorm of x (or of the layer's input: parallel residual); w1; gelu(+ b1); w2
       HIP_TRY(timed(e, HE_K_NORM, (double)m * dim * (8 + 1 + 0.125) + dim * 8.0, [&] {
         return launch_layernorm_quant(e->xq, e->xs, nullptr, nullptr, c.parallel_residual ? e->before : e->x,
                                       e->vec(HE_T_RMS_FFN, (int64_t)l * dim), e->vec(HE_T_LN_FFN_BIAS, (int64_t)l * dim),
                                       m, dim, dim, W, W / 32, 0, e->bias, s);
       }));
+      const float *b1 = e->vec(HE_T_B1, (int64_t)l * hidden);
+      if (ffn_in_gemm(e, m)) {
+        const MatSeg w1[1] = {{e->mat(HE_T_W1, l), e->mat_scales(HE_T_W1, l), e->hb, hidden, hidden, 0, b1}};
+        HIP_TRY(timed(e, HE_K_GEMM, matmul_bytes(e, w1, 1, dim, m),
+                      [&] { return gemm_ffn_launch(e, w1, 1, dim, m, e->xq, e->xs, gq, e->hb2); }));
+        HIP_TRY(matmul(e, w2, 1, hidden, m, gq, e->hb2));
+        continue;
+      }
       const MatSeg w1[1] = {{e->mat(HE_T_W1, l), e->mat_scales(HE_T_W1, l), e->hb, hidden, hidden, 0}};
       HIP_TRY(matmul(e, w1, 1, dim, m, e->xq, e->xs));
       HIP_TRY(timed(e, HE_K_ELEMENTWISE, (double)m * hidden * (8 + 1 + 0.125), [&] {
-        return launch_gelu_quant(e->xq, e->xs, nullptr, e->hb, e->vec(HE_T_B1, (int64_t)l * hidden), m, hidden,
-                                 hidden, W, W / 32, e->bias, s);
+        return launch_gelu_quant(e->xq, e->xs, nullptr, e->hb, b1, m, hidden, hidden, W, W / 32, e->bias, s);
       }));
-      const MatSeg w2g[1] = {{e->mat(HE_T_W2, l), e->mat_scales(HE_T_W2, l), e->x, dim, dim, 1}};
-      HIP_TRY(matmul(e, w2g, 1, hidden, m, e->xq, e->xs));
-      HIP_TRY(timed(e, HE_K_ELEMENTWISE, (double)m * dim * 12,
-                    [&] { return launch_add_rows(e->x, e->vec(HE_T_B2, (int64_t)l * dim), m, dim, dim, s); }));
+      HIP_TRY(matmul(e, w2, 1, hidden, m, e->xq, e->xs));
       continue;
     }
     const MatSeg w13[2] = {{e->mat(HE_T_W1, l), e->mat_scales(HE_T_W1, l), e->hb, hidden, hidden, 0},
@@ -772,14 +786,9 @@ int32_t run_chunk(he_engine *e, const int32_t *tokens, int32_t m, int32_t pos0, 
                                     W, W / 32, 0, c.rms_norm_eps, e->bias, s, &f13);
       }));
     }
-    const MatSeg w2[1] = {{e->mat(HE_T_W2, l), e->mat_scales(HE_T_W2, l), e->x, dim, dim, 1}};
-    if (glu_in_gemm(e, m)) {
-      // the GEMM finishes the SwiGLU and its quantize_x itself; its bytes and scales go where h1 and h3 would (hb and
-      // hb2 hold [chunk][W] bytes and [chunk][W / 32] floats: glu_in_gemm checks), apart from the w1 / w3 GEMM's
-      // input in xq / xs
-      int8_t *gq = reinterpret_cast<int8_t *>(e->hb);
+    if (ffn_in_gemm(e, m)) {
       HIP_TRY(timed(e, HE_K_GEMM, matmul_bytes(e, w13, 2, dim, m),
-                    [&] { return gemm_glu_launch(e, w13, dim, m, e->xq, e->xs, gq, e->hb2); }));
+                    [&] { return gemm_ffn_launch(e, w13, 2, dim, m, e->xq, e->xs, gq, e->hb2); }));
       HIP_TRY(matmul(e, w2, 1, hidden, m, gq, e->hb2));
       continue;
     }

@@ -1,7 +1,6 @@
 // forms.hip — the kernels of the model forms beside the Llama/Qwen2 one, each in the reference's float32 order:
 //   layernorm (kernels/kernel.ts:610-634) then quantize_x: GPT-2 and GPT-NeoX (public/forward.js:1031,1063,1082);
 //   gelu with the bias of w1 (kernels/kernel.ts:636-652) then quantize_x;
-//   the biases added after wo and w2 (add_inplace, kernels/kernel.ts:691-693; public/forward.js:1061,1070-1071);
 //   Qwen3's q/k head norms: rmsnorm (kernels/kernel.ts:330-342) over every head of q and k after the biases
 //   (public/forward.js:1038-1047);
 //   the outlier channels of the classifier's input (public/forward.js:801-812,1084-1089): their float32 columns of the
@@ -89,15 +88,6 @@ __global__ __launch_bounds__(256) void gelu_quant_kernel(int8_t *xq, float *xs, 
   const float o = v / (1.0f + vexp(-2.0f * inner));
   if (out) out[(int64_t)t * h_stride + j] = o;
   quantize_group(o, xq + (int64_t)t * xq_stride, xs + (int64_t)t * xs_stride, j, g, bias);
-}
-
-// x[t][j] = f32(x[t][j] + b[j])
-__global__ __launch_bounds__(256) void add_rows_kernel(float *x, const float *b, int32_t n, int32_t stride) {
-  const int t = blockIdx.y;
-  for (int j = blockIdx.x * 256 + threadIdx.x; j < n; j += gridDim.x * 256) {
-    float *p = x + (int64_t)t * stride + j;
-    *p = *p + b[j];
-  }
 }
 
 // Qwen3: every head of q and k (a wave each): + its bias where given, then rmsnorm over the head's hs values in place
@@ -213,12 +203,6 @@ hipError_t launch_gelu_quant(int8_t *xq, float *xs, float *out, const float *h, 
   const int64_t groups = (int64_t)m * (n / GS);
   hipLaunchKernelGGL(gelu_quant_kernel, dim3((unsigned)((groups + 7) / 8)), dim3(256), 0, s, xq, xs, out, h, b, m, n,
                      h_stride, xq_stride, xs_stride, bias);
-  return hipGetLastError();
-}
-
-hipError_t launch_add_rows(float *x, const float *b, int32_t m, int32_t n, int32_t stride, hipStream_t s) {
-  const int blocks = std::min(64, (n + 255) / 256);
-  hipLaunchKernelGGL(add_rows_kernel, dim3(blocks, m), dim3(256), 0, s, x, b, n, stride);
   return hipGetLastError();
 }
 

@@ -341,8 +341,10 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2))) void ge
       float *y = (si == 2 ? a.seg[2].y : si == 1 ? a.seg[1].y : a.seg[0].y);
       const int stride = (si == 2 ? a.seg[2].y_stride : si == 1 ? a.seg[1].y_stride : a.seg[0].y_stride);
       const int accumulate = (si == 2 ? a.seg[2].accumulate : si == 1 ? a.seg[1].accumulate : a.seg[0].accumulate);
+      const float *bias = (si == 2 ? a.seg[2].bias : si == 1 ? a.seg[1].bias : a.seg[0].bias);
       float *dst = y + (int64_t)t * stride + r;
-      *dst = accumulate ? *dst + out[h][v] : out[h][v];
+      const float o = accumulate ? *dst + out[h][v] : out[h][v];
+      *dst = bias ? o + bias[r] : o;
     }
   }
 }
@@ -352,6 +354,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2))) void ge
 hipError_t launch_gemm(const MatArgs &a, bool six, bool relaxed, hipStream_t s) {
   if (a.m < 1 || a.total_rows < 1 || a.k < 32 || a.k % 32) return hipErrorInvalidValue;
   if (a.sums && (a.nseg != 1 || !relaxed)) return hipErrorInvalidValue;
+  if (a.qkv.on && (a.sums || a.nseg != 3 || !gemm_finishes(a.total_rows, a.m, relaxed))) return hipErrorInvalidValue;
   if (!a.sums && (!relaxed || gemm_chains_faster(a.total_rows, a.m, false))) return launch_gemm_chains(a, six, relaxed, s);
   const int64_t blocks = (int64_t)((a.total_rows + BR - 1) / BR) * ((a.m + BT - 1) / BT);
   if (blocks > (1ll << 30)) return hipErrorInvalidValue;
@@ -370,15 +373,25 @@ hipError_t launch_gemm(const MatArgs &a, bool six, bool relaxed, hipStream_t s) 
   return hipGetLastError();
 }
 
+bool gemm_finishes(int32_t rows, int32_t m, bool relaxed) { return !relaxed || gemm_chains_faster(rows, m, false); }
+
+// a quantized output of `hidden` units: its 4-byte runs and its scales aligned and inside [m][q_stride] / [m][s_stride]
+static bool takes_units(const GluOut &g, int32_t hidden) {
+  return hidden >= 32 && hidden % 32 == 0 && g.q && g.s && (g.bias == 0 || g.bias == 64) && g.q_stride >= hidden &&
+         g.q_stride % 4 == 0 && g.s_stride >= hidden / 32 && reinterpret_cast<uintptr_t>(g.q) % 4 == 0;
+}
+
+hipError_t launch_gemm_gelu(const MatArgs &a, bool six, bool relaxed, hipStream_t s) {
+  if (a.m < 1 || a.nseg != 1 || a.sums || a.k < 32 || a.k % 32 || !a.seg[0].bias || a.total_rows != a.seg[0].rows ||
+      !takes_units(a.glu, a.total_rows) || !gemm_finishes(a.total_rows, a.m, relaxed))
+    return hipErrorInvalidValue;
+  return launch_gemm_chains_gelu(a, six, relaxed, s);
+}
+
 hipError_t launch_gemm_glu(const MatArgs &a, bool six, bool relaxed, hipStream_t s) {
-  const GluOut &g = a.glu;
   if (a.m < 1 || a.nseg != 2 || a.sums || a.k < 32 || a.k % 32) return hipErrorInvalidValue;
   const int hidden = a.seg[0].rows;
-  if (hidden < 32 || hidden % 32 || a.seg[1].rows != hidden || a.total_rows != 2 * hidden) return hipErrorInvalidValue;
-  // the output's 4-byte runs and its scales: every store aligned and inside [m][q_stride] / [m][s_stride]
-  if (!g.q || !g.s || (g.bias != 0 && g.bias != 64) || g.q_stride < hidden || g.q_stride % 4 ||
-      g.s_stride < hidden / 32 || reinterpret_cast<uintptr_t>(g.q) % 4)
-    return hipErrorInvalidValue;
+  if (!takes_units(a.glu, hidden) || a.seg[1].rows != hidden || a.total_rows != 2 * hidden) return hipErrorInvalidValue;
   if (!relaxed || gemm_chains_faster(a.total_rows, a.m, true)) return launch_gemm_chains_glu(a, six, relaxed, s);
   const int64_t blocks = (int64_t)(hidden / 32) * ((a.m + BT - 1) / BT);
   if (blocks > (1ll << 30)) return hipErrorInvalidValue;

@@ -31,6 +31,10 @@ typedef int v4i __attribute__((ext_vector_type(4)));
 constexpr int MAGIC = 0x4B400000;
 constexpr float MAGIC_F = 12582912.0f;
 
+// what a block does with its outputs: stores them (or finishes q / k / v: a.qkv), or finishes the FFN's activation and its
+// quantize_x (a.glu)
+enum { EPI_STORE = 0, EPI_GLU, EPI_GELU };
+
 // quantize_x(bias 0)'s lane sums: the 16 bytes of half a group as the four words of lane sums 0..3 (word k: bytes 2k,
 // 2k + 1, 2k + 8, 2k + 9)
 __device__ __forceinline__ void lane_words(uint4 v, uint32_t (&o)[4]) {
@@ -40,7 +44,46 @@ __device__ __forceinline__ void lane_words(uint4 v, uint32_t (&o)[4]) {
   o[3] = __builtin_amdgcn_perm(v.w, v.y, 0x07060302u);
 }
 
-template <bool SIX, bool PLAIN, int RT, int TT, int RB, int CK, int D, bool GLU>
+// four rows (row, row + 1, .. of the launch's q, k and v rows, all of one segment: every segment is whole heads) of token t
+// finished as qkv_post_kernel does: + bias, RoPE's two pairs of q and k, q stored, k and v into the cache
+__device__ __forceinline__ void finish_qkv(const MatArgs &a, int row, int t, const float (&s)[4]) {
+  if (row >= a.total_rows) return;
+  const QkvFuse &f = a.qkv;
+  const int n0 = a.seg[0].rows, n1 = a.seg[1].rows;
+  const int seg = row < n0 ? 0 : (row < n0 + n1 ? 1 : 2), r = row - (seg == 0 ? 0 : (seg == 1 ? n0 : n0 + n1));
+  const int pos = (f.dpos ? *f.dpos : f.pos) + t;
+  const float *bias = seg == 0 ? f.bq : (seg == 1 ? f.bk : f.bv);
+  float v[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) v[j] = bias ? s[j] + bias[r + j] : s[j];
+  if (seg < 2) {
+#pragma unroll
+    for (int j = 0; j < 4; j += 2) {
+      const int at = (r + j) % f.hs;
+      if (at < f.rot) {
+        const float c = f.cos_t[(int64_t)pos * (f.hs / 2) + at / 2], sn = f.sin_t[(int64_t)pos * (f.hs / 2) + at / 2];
+        const float v0 = v[j], v1 = v[j + 1];
+        v[j] = v0 * c - v1 * sn;
+        v[j + 1] = v0 * sn + v1 * c;
+      }
+    }
+  }
+  if (seg == 0) {
+    float *y = a.seg[0].y + (int64_t)t * a.seg[0].y_stride + r;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) y[j] = v[j];
+    return;
+  }
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int64_t at = seg == 1 ? (int64_t)pos * f.kvdim + r + j : (int64_t)(r + j) * f.vstride + pos;
+    void *cache = seg == 1 ? f.kcache : f.vcache;
+    if (f.half) reinterpret_cast<uint16_t *>(cache)[at] = to_f16(v[j]);
+    else reinterpret_cast<float *>(cache)[at] = v[j];
+  }
+}
+
+template <bool SIX, bool PLAIN, int RT, int TT, int RB, int CK, int D, int EPI>
 struct Chains {
   static constexpr int NT = 256 * RB;                    // threads
   static constexpr int PITCH = CK * 32 + 16;  // LDS bytes of a row of a stage: 16 rows' 8-byte reads fall on distinct banks
@@ -61,10 +104,12 @@ struct Chains {
   };
 };
 
-template <bool SIX, bool PLAIN, int RT, int TT, int RB, int CK, int D, bool GLU>
+template <bool SIX, bool PLAIN, int RT, int TT, int RB, int CK, int D, int EPI>
 __global__ __launch_bounds__(256 * RB) __attribute__((amdgpu_waves_per_eu(2))) void gemm_chains_kernel(const MatArgs a) {
-  using P = Chains<SIX, PLAIN, RT, TT, RB, CK, D, GLU>;
+  using P = Chains<SIX, PLAIN, RT, TT, RB, CK, D, EPI>;
+  constexpr bool GLU = EPI == EPI_GLU;
   static_assert(!GLU || (RB == 2 && RT == 2), "the SwiGLU's blocks are 32 units of w1 and of w3");
+  static_assert(EPI != EPI_GELU || RB * RT == 2, "the GELU's blocks are 32 units");
   constexpr int NT = P::NT, PITCH = P::PITCH;
   extern __shared__ float4 lds4[];
   uint8_t *const lds = reinterpret_cast<uint8_t *>(lds4);
@@ -349,6 +394,28 @@ __global__ __launch_bounds__(256 * RB) __attribute__((amdgpu_waves_per_eu(2))) v
     }
     return;
   }
+  if constexpr (EPI == EPI_GELU) {
+    // a token's 8 quads of the block's 32 units are 8 lanes already: gelu(h + b) as gelu_quant_kernel computes it, then
+    // quantize_x of the token's group
+#pragma unroll
+    for (int i = 0; i < (PER + NT - 1) / NT; ++i) {
+      int quad, token;
+      piece(i, &quad, &token);
+      const int t = t0 + token;
+      if ((PER % NT != 0 && tid + NT * i >= PER) || t >= a.m) continue;  // (a token's 8 lanes leave together)
+      const float *b = a.seg[0].bias + r0 + 4 * quad;
+      const float h[4] = {sum[i].x + b[0], sum[i].y + b[1], sum[i].z + b[2], sum[i].w + b[3]};
+      float o[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float inner = 0.7978845608028654f * (h[j] + ((0.044715f * h[j]) * h[j]) * h[j]);
+        o[j] = h[j] / (1.0f + vexp(-2.0f * inner));
+      }
+      quantize_group4(make_float4(o[0], o[1], o[2], o[3]), a.glu.q + (int64_t)t * a.glu.q_stride,
+                      a.glu.s + (int64_t)t * a.glu.s_stride, r0 + 4 * quad, r0 / 32, a.glu.bias);
+    }
+    return;
+  }
 #pragma unroll
   for (int i = 0; i < (PER + NT - 1) / NT; ++i) {
     int quad, token;
@@ -356,15 +423,22 @@ __global__ __launch_bounds__(256 * RB) __attribute__((amdgpu_waves_per_eu(2))) v
     const int t = t0 + token, row = r0 + 4 * quad;
     if ((PER % NT != 0 && tid + NT * i >= PER) || t >= a.m) continue;
     const float v[4] = {sum[i].x, sum[i].y, sum[i].z, sum[i].w};
-    auto place = [&](int r, int *accumulate) {
+    if (a.qkv.on) {  // uniform
+      finish_qkv(a, row, t, v);
+      continue;
+    }
+    auto place = [&](int r, int *accumulate, const float **bias) {
       const bool third = a.nseg > 2 && r >= n0 + n1, second = a.nseg > 1 && r >= n0;
+      const float *b = third ? a.seg[2].bias : (second ? a.seg[1].bias : a.seg[0].bias);
+      *bias = b ? b + (r - (third ? n0 + n1 : (second ? n0 : 0))) : nullptr;
       float *y = third ? a.seg[2].y : (second ? a.seg[1].y : a.seg[0].y);
       const int stride = third ? a.seg[2].y_stride : (second ? a.seg[1].y_stride : a.seg[0].y_stride);
       *accumulate = third ? a.seg[2].accumulate : (second ? a.seg[1].accumulate : a.seg[0].accumulate);
       return y + (int64_t)t * stride + (r - (third ? n0 + n1 : (second ? n0 : 0)));
     };
     int accumulate;
-    float *const dst = place(min(row, a.total_rows - 1), &accumulate);
+    const float *bias;
+    float *const dst = place(min(row, a.total_rows - 1), &accumulate, &bias);
     if (row + 3 < a.total_rows && ((n0 | n1) & 3) == 0 && (reinterpret_cast<uintptr_t>(dst) & 15) == 0) {
       // the four rows lie in one segment, side by side on 16 bytes
       float4 o = make_float4(v[0], v[1], v[2], v[3]);
@@ -372,34 +446,36 @@ __global__ __launch_bounds__(256 * RB) __attribute__((amdgpu_waves_per_eu(2))) v
         const float4 y4 = *reinterpret_cast<const float4 *>(dst);
         o = make_float4(y4.x + v[0], y4.y + v[1], y4.z + v[2], y4.w + v[3]);
       }
+      if (bias) o = make_float4(o.x + bias[0], o.y + bias[1], o.z + bias[2], o.w + bias[3]);
       *reinterpret_cast<float4 *>(dst) = o;
     } else {
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         if (row + j >= a.total_rows) break;
-        float *const d = place(row + j, &accumulate);
-        *d = accumulate ? *d + v[j] : v[j];
+        float *const d = place(row + j, &accumulate, &bias);
+        const float o = accumulate ? *d + v[j] : v[j];
+        *d = bias ? o + *bias : o;
       }
     }
   }
 }
 
-template <bool SIX, bool PLAIN, int RT, int TT, int RB, int CK, int D, bool GLU>
+template <bool SIX, bool PLAIN, int RT, int TT, int RB, int CK, int D, int EPI>
 hipError_t launch_one(const MatArgs &a, hipStream_t s) {
-  using P = Chains<SIX, PLAIN, RT, TT, RB, CK, D, GLU>;
-  const int rows = GLU ? 2 * a.seg[0].rows : a.total_rows;
+  using P = Chains<SIX, PLAIN, RT, TT, RB, CK, D, EPI>;
+  const int rows = a.total_rows;
   const int64_t blocks = (int64_t)((rows + P::ROWS - 1) / P::ROWS) * ((a.m + P::TOKENS - 1) / P::TOKENS);
   if (blocks > (1ll << 30)) return hipErrorInvalidValue;
   if (P::LDS > 64 * 1024) {
     static bool sized = false;  // once a process: let the kernel take LDS past 64 KiB
     if (!sized) {
-      const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_chains_kernel<SIX, PLAIN, RT, TT, RB, CK, D, GLU>),
+      const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_chains_kernel<SIX, PLAIN, RT, TT, RB, CK, D, EPI>),
                                                hipFuncAttributeMaxDynamicSharedMemorySize, P::LDS);
       if (e != hipSuccess) return e;
       sized = true;
     }
   }
-  hipLaunchKernelGGL((gemm_chains_kernel<SIX, PLAIN, RT, TT, RB, CK, D, GLU>), dim3((unsigned)blocks), dim3(P::NT), P::LDS, s, a);
+  hipLaunchKernelGGL((gemm_chains_kernel<SIX, PLAIN, RT, TT, RB, CK, D, EPI>), dim3((unsigned)blocks), dim3(P::NT), P::LDS, s, a);
   return hipGetLastError();
 }
 
@@ -416,9 +492,9 @@ int64_t tiles(int64_t n, int64_t size) { return (n + size - 1) / size; }
 template <bool SIX, bool PLAIN>
 hipError_t launch_tile(const MatArgs &a, hipStream_t s) {
   const int64_t rows = a.total_rows, m = a.m;
-  if (m <= 16 || tiles(rows, 16) * tiles(m, 16) <= 2 * CUS) return launch_one<SIX, PLAIN, 1, 1, 1, 16, 2, false>(a, s);
-  if (tiles(rows, 32) * tiles(m, 32) <= CUS) return launch_one<SIX, PLAIN, 1, 2, 2, 16, 2, false>(a, s);
-  return launch_one<SIX, PLAIN, 2, 2, 2, 8, 2, false>(a, s);
+  if (m <= 16 || tiles(rows, 16) * tiles(m, 16) <= 2 * CUS) return launch_one<SIX, PLAIN, 1, 1, 1, 16, 2, EPI_STORE>(a, s);
+  if (tiles(rows, 32) * tiles(m, 32) <= CUS) return launch_one<SIX, PLAIN, 1, 2, 2, 16, 2, EPI_STORE>(a, s);
+  return launch_one<SIX, PLAIN, 2, 2, 2, 8, 2, EPI_STORE>(a, s);
 }
 
 // the SwiGLU's blocks (32 units of w1 and of w3): 16 tokens while that is at most one block a CU (4096 rows of K 512, 64
@@ -427,9 +503,18 @@ hipError_t launch_tile(const MatArgs &a, hipStream_t s) {
 template <bool SIX, bool PLAIN>
 hipError_t launch_glu_tile(const MatArgs &a, hipStream_t s) {
   const int64_t units = tiles(a.seg[0].rows, 32), m = a.m;
-  if (m <= 16 || units * tiles(m, 16) <= CUS) return launch_one<SIX, PLAIN, 2, 1, 2, 8, 2, true>(a, s);
-  if (tiles(m, 16) == 3) return launch_one<SIX, PLAIN, 2, 3, 2, 8, 2, true>(a, s);
-  return launch_one<SIX, PLAIN, 2, 2, 2, 8, 2, true>(a, s);
+  if (m <= 16 || units * tiles(m, 16) <= CUS) return launch_one<SIX, PLAIN, 2, 1, 2, 8, 2, EPI_GLU>(a, s);
+  if (tiles(m, 16) == 3) return launch_one<SIX, PLAIN, 2, 3, 2, 8, 2, EPI_GLU>(a, s);
+  return launch_one<SIX, PLAIN, 2, 2, 2, 8, 2, EPI_GLU>(a, s);
+}
+
+// the GELU's blocks (32 units): the tiles of launch_tile that hold a whole group
+template <bool SIX, bool PLAIN>
+hipError_t launch_gelu_tile(const MatArgs &a, hipStream_t s) {
+  const int64_t units = tiles(a.total_rows, 32), m = a.m;
+  if (m <= 16) return launch_one<SIX, PLAIN, 1, 1, 2, 16, 2, EPI_GELU>(a, s);
+  if (units * tiles(m, 32) <= CUS) return launch_one<SIX, PLAIN, 1, 2, 2, 16, 2, EPI_GELU>(a, s);
+  return launch_one<SIX, PLAIN, 1, 2, 2, 8, 2, EPI_GELU>(a, s);
 }
 
 }  // namespace
@@ -455,6 +540,11 @@ hipError_t launch_gemm_chains(const MatArgs &a, bool six, bool relaxed, hipStrea
 hipError_t launch_gemm_chains_glu(const MatArgs &a, bool six, bool relaxed, hipStream_t s) {
   if (six) return relaxed ? launch_glu_tile<true, false>(a, s) : launch_glu_tile<true, true>(a, s);
   return relaxed ? launch_glu_tile<false, false>(a, s) : launch_glu_tile<false, true>(a, s);
+}
+
+hipError_t launch_gemm_chains_gelu(const MatArgs &a, bool six, bool relaxed, hipStream_t s) {
+  if (six) return relaxed ? launch_gelu_tile<true, false>(a, s) : launch_gelu_tile<true, true>(a, s);
+  return relaxed ? launch_gelu_tile<false, false>(a, s) : launch_gelu_tile<false, true>(a, s);
 }
 
 }  // namespace ple

@@ -48,13 +48,15 @@ struct RowAt {
   const float *ws;
   float *y;
   int32_t r, y_stride, accumulate;
+  const float *bias;
 };
 __device__ __forceinline__ RowAt row_at(const MatArgs &a, int row) {
   const int n0 = a.seg[0].rows, n1 = a.seg[1].rows;
   if (a.nseg > 2 && row >= n0 + n1)
-    return {a.seg[2].w, a.seg[2].ws, a.seg[2].y, row - n0 - n1, a.seg[2].y_stride, a.seg[2].accumulate};
-  if (a.nseg > 1 && row >= n0) return {a.seg[1].w, a.seg[1].ws, a.seg[1].y, row - n0, a.seg[1].y_stride, a.seg[1].accumulate};
-  return {a.seg[0].w, a.seg[0].ws, a.seg[0].y, row, a.seg[0].y_stride, a.seg[0].accumulate};
+    return {a.seg[2].w, a.seg[2].ws, a.seg[2].y, row - n0 - n1, a.seg[2].y_stride, a.seg[2].accumulate, a.seg[2].bias};
+  if (a.nseg > 1 && row >= n0) return {a.seg[1].w, a.seg[1].ws, a.seg[1].y, row - n0, a.seg[1].y_stride, a.seg[1].accumulate,
+            a.seg[1].bias};
+  return {a.seg[0].w, a.seg[0].ws, a.seg[0].y, row, a.seg[0].y_stride, a.seg[0].accumulate, a.seg[0].bias};
 }
 
 // the decode paths' store of row `row`'s result: y = sum (or y + sum). With a.qkv on (every lane of the wave calls
@@ -64,7 +66,10 @@ __device__ __forceinline__ void store_row(const MatArgs &a, int row, float sum, 
   const RowAt at = row_at(a, min(row, a.total_rows - 1));
   float *y = at.y + at.r;
   if (!a.qkv.on) {
-    if (valid) *y = at.accumulate ? *y + sum : sum;
+    if (valid) {
+      const float o = at.accumulate ? *y + sum : sum;
+      *y = at.bias ? o + at.bias[at.r] : o;
+    }
     return;
   }
   // (every field read by value: a reference into the kernel's argument struct makes the compiler copy it to scratch)
@@ -72,14 +77,14 @@ __device__ __forceinline__ void store_row(const MatArgs &a, int row, float sum, 
   void *kcache = a.qkv.kcache, *vcache = a.qkv.vcache;
   const int32_t *dpos = a.qkv.dpos;
   const int pos = dpos ? *dpos : a.qkv.pos, hs = a.qkv.hs, kvdim = a.qkv.kvdim, half = a.qkv.half;
-  const int vstride = a.qkv.vstride;
+  const int vstride = a.qkv.vstride, rot = a.qkv.rot;
   const int n0 = a.seg[0].rows, n1 = a.seg[1].rows;
   const int seg = row < n0 ? 0 : (row < n0 + n1 ? 1 : 2), r = at.r;
   const float *bias = seg == 0 ? bq : (seg == 1 ? bk : bv);
   const float v = bias ? sum + bias[r] : sum;
   const float partner = dpp_xor1(v);  // the pair's other row (lanes 2i, 2i + 1)
   float o = v;
-  if (seg < 2) {
+  if (seg < 2 && r % hs < rot) {  // (a pair's two rows take the branch together)
     const int ci = (r % hs) >> 1;
     const float c = cos_t[(int64_t)pos * (hs / 2) + ci], s = sin_t[(int64_t)pos * (hs / 2) + ci];
     const bool even = (r & 1) == 0;
@@ -240,7 +245,8 @@ __global__ __launch_bounds__(256) void gemv_kernel(const MatArgs a) {
       for (int g = G4; g < G; ++g) sum = sum + tl[g - G4];
     }
     float *y = sg.y + (int64_t)lane * sg.y_stride + r;
-    *y = sg.accumulate ? *y + sum : sum;
+    const float o = sg.accumulate ? *y + sum : sum;
+    *y = sg.bias ? o + sg.bias[r] : o;
   }
 }
 

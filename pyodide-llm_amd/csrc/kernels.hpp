@@ -9,7 +9,7 @@ namespace ple {
 
 // one matrix of a GEMV/GEMM launch: rows [rows][K] int8 (or int6 groups of 24 bytes), scales [rows][K/32]; the
 // output y[t * y_stride + r] for token t, row r (accumulate: y = y + result, the residual add of kernels/kernel.ts:
-// 691-693 fused)
+// 691-693 fused; bias: then + bias[r], GPT-2's and GPT-NeoX's add after it)
 struct MatSeg {
   const uint8_t *w;
   const float *ws;
@@ -17,21 +17,24 @@ struct MatSeg {
   int32_t rows;
   int32_t y_stride;
   int32_t accumulate;
+  const float *bias;
 };
 
 // the value cache holds a column's positions side by side, each column seq_len rounded up to 64 positions (256 bytes
 // of float32): the weighted sums read a column's values as contiguous runs
 inline int32_t value_stride(int32_t seq_len) { return (seq_len + 63) & ~63; }
 
-// one token's q / k / v matmul (three segments) finishing the token's attention inputs in its epilogue, as
-// launch_qkv_post does (the bias add, RoPE on q and k, k and v into the cache): the decode path only, rows in pairs
+// the q / k / v matmul (three segments) finishing the tokens' attention inputs in its epilogue, as launch_qkv_post does
+// (the bias add, RoPE on q and k, k and v into the cache; k and v go nowhere else): the one-token decode path, and the
+// GEMM where gemm_finishes()
 struct QkvFuse {
   int32_t on;
   const float *bq, *bk, *bv;   // Qwen2 biases or null
   const float *cos_t, *sin_t;  // [seq_len][hs/2]
   void *kcache, *vcache;       // this layer's keys [seq_len][kv_dim] and values [kv_dim][vstride]
   int32_t pos, hs, kvdim, half, vstride;
-  const int32_t *dpos;  // the position in device memory (a replayed decode step), or null: pos
+  const int32_t *dpos;  // the first position in device memory (a replayed decode step), or null: pos
+  int32_t rot;          // the values of each head RoPE turns: hs all, 0 none
 };
 
 // An L2 fill ahead of a one-token GEMV, run by extra blocks of the rmsnorm launch before it, which leaves most CUs and
@@ -78,7 +81,7 @@ struct MatArgs {
   // one token, rows of 1-4 KiB (decode_persistent): the persistent GEMV, about one block a CU that loops over its
   // rows (no L2Fetch fits it: its blocks take rows in another order)
   int32_t persistent;
-  GluOut glu;  // launch_gemm_glu only
+  GluOut glu;  // launch_gemm_glu and launch_gemm_gelu only
 };
 
 // rows a block of the one-token decode GEMV takes (launch_gemv with m = 1, bias 64, no sums) for rows of k, 0 where
@@ -102,11 +105,17 @@ int32_t gemv_tokens(int32_t k, bool relaxed);
 hipError_t launch_gemm(const MatArgs &a, bool six, bool relaxed, hipStream_t s);
 // the w1 / w3 GEMM with the SwiGLU and its quantize_x in the epilogue (a.glu)
 hipError_t launch_gemm_glu(const MatArgs &a, bool six, bool relaxed, hipStream_t s);
+// the w1 GEMM of GPT-2's and GPT-NeoX's layer with gelu(. + bias) (seg[0].bias) and its quantize_x in the epilogue
+// (a.glu); where gemm_finishes()
+hipError_t launch_gemm_gelu(const MatArgs &a, bool six, bool relaxed, hipStream_t s);
+// whether the GEMM of m tokens against `rows` rows in all takes a.qkv, and whether launch_gemm_gelu takes it
+bool gemm_finishes(int32_t rows, int32_t m, bool relaxed);
 // gemm_chains.hip: the GEMM with each float32 lane chain on a wave of its own, for bias 0 and for the grids where it is
 // the faster one (rows: of every segment). launch_gemm and launch_gemm_glu check the arguments and choose.
 bool gemm_chains_faster(int32_t rows, int32_t m, bool glu);
 hipError_t launch_gemm_chains(const MatArgs &a, bool six, bool relaxed, hipStream_t s);
 hipError_t launch_gemm_chains_glu(const MatArgs &a, bool six, bool relaxed, hipStream_t s);
+hipError_t launch_gemm_chains_gelu(const MatArgs &a, bool six, bool relaxed, hipStream_t s);
 
 // quantize_x over m rows of n (x_stride apart) into xq (xq_stride) / xs (xs_stride)
 hipError_t launch_quantize(int8_t *xq, float *xs, const float *x, int32_t m, int32_t n, int32_t x_stride,
@@ -158,7 +167,7 @@ struct AttnArgs {
   // the first position in device memory (a replayed decode step), or null: pos0; with it, pos0 is only the largest
   // first position the launch may see (grid and LDS sizes)
   const int32_t *dpos;
-  // where attention_quantizes(): quantize_x(bias) of out as well, [m][xq_stride] and [m][xs_stride] (null: not)
+  // where attention_quantizes(): quantize_x(bias) of out, [m][xq_stride] and [m][xs_stride] (null: out only)
   int8_t *xq;
   float *xs;
   int32_t xq_stride, xs_stride, bias;
@@ -175,8 +184,8 @@ bool attention_supported(int32_t hs, int32_t nh, int32_t nkv);
 // the longest context (a multiple of 4) the attention kernels take: a (token, head)'s exponentials are held in one
 // block's LDS (160 KiB on gfx950) for their ordered sum
 int32_t attention_most_positions();
-// whether launch_attention writes quantize_x of its output too (a.xq): decode launches whose head size is a multiple
-// of 32 (a block holds a whole group) and whose context fits the decode kernel's LDS
+// whether launch_attention takes a.xq and writes quantize_x of its output (the prompt's kernels: in place of a.out): head
+// sizes that are a multiple of 32 (a block holds a whole group)
 bool attention_quantizes(const AttnArgs &a);
 
 // a streaming read of bytes (a multiple of 16) at p in launch shape `shape` (0 .. read_ceiling_shapes() - 1: loads a
@@ -285,8 +294,6 @@ hipError_t launch_layernorm_quant(int8_t *xq, float *xs, float *out, float *copy
 // gelu(h + b) then quantize_x, m tokens (n a multiple of 32)
 hipError_t launch_gelu_quant(int8_t *xq, float *xs, float *out, const float *h, const float *b, int32_t m, int32_t n,
                              int32_t h_stride, int32_t xq_stride, int32_t xs_stride, int32_t bias, hipStream_t s);
-// x[t][j] += b[j] for m rows of n, stride apart
-hipError_t launch_add_rows(float *x, const float *b, int32_t m, int32_t n, int32_t stride, hipStream_t s);
 // Qwen3: q and k heads + bias (optional), then RMS-normalized in place by qw / kw (hs values each)
 hipError_t launch_head_norm(float *q, float *k, const float *bq, const float *bk, const float *qw, const float *kw,
                             int32_t m, int32_t nh, int32_t nkv, int32_t hs, int32_t q_stride, int32_t kv_stride,

@@ -57,3 +57,24 @@ def test_swiglu_epilogue_bits(hidden, m, six, relaxed):
     assert same_bits(kv["keys"], k.reshape(-1)) and same_bits(kv["values"], v.reshape(-1))
     eng.release()
     ref.close()
+
+
+@pytest.mark.parametrize("arch,m", [("gpt2", 17), ("neox", 100), ("gpt2", 1024)])
+def test_layer_norm_forms_epilogues(arch, m):
+    """GPT-2's and GPT-NeoX's prompt layer: q/k/v finished in the GEMM (no rotation; part of each head turned), the biases
+    after wo and w2, the GELU in the GEMM and, in a grid that the 64 x 128 blocks take (1024 tokens), on its own"""
+    extra = dict(rotary=16, parallel_residual=1) if arch == "neox" else {}
+    cfg = ol.config(dim=768, hidden_dim=3072, n_layers=2, n_heads=12, n_kv_heads=12, head_size=64, vocab_size=64,
+                    seq_len=1024, shared_classifier=1, half_kv=1, arch=arch, **extra)
+    tensors, size = ol.places(cfg)
+    ck = ol.vary_vectors(cfg, tensors, ol.synth_checkpoint(cfg, tensors, size, seed=8), seed=9)
+    cos, sin = package().rope_tables(cfg.seq_len, cfg.head_size, 10000.0, cfg.rotary)
+    tokens = [int(t) for t in np.random.default_rng(m).integers(0, cfg.vocab_size, size=m)]
+    ref = ol.Model(cfg, tensors, ck, cos, sin, max_block=1024)
+    eng = package().open_config(cfg, tensors, ck, cos, sin, max_block=1024)
+    ref.run(tokens, 0, False)
+    eng.forwardMany(tokens, 0)
+    kv, (k, v) = eng.keysAndValues(0, m), ref.kv(0, m)
+    assert same_bits(kv["keys"], k.reshape(-1)) and same_bits(kv["values"], v.reshape(-1))
+    eng.release()
+    ref.close()
