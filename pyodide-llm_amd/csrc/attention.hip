@@ -421,6 +421,120 @@ __global__ __launch_bounds__(A2_NT) void attend2_kernel(const AttnArgs a) {
   }
 }
 
+// The whole of a decode attention in one launch, for contexts of up to A1_MOST positions: one block of 1024 threads a
+// (token, query head, 16 columns), as attend2_kernel, that makes the head's scores itself, a thread a position. The head's
+// other column blocks repeat them (A1_SCORES bounds the keys a block reads), which costs less than the scores' launch
+// where everything fits the caches. Then the maximum over the block, and attend2_kernel's steps with a thread a
+// (four-position block, 4 columns), its values requested with the keys. Bound by latency: the loads, two ordered sums of
+// count / 4 steps, five barriers. (With the FFN's activation in w2's GEMV: two launches a layer fewer; a sampled step of
+// the 15M shape 230 -> 203 us.)
+constexpr int A1_MOST = 1024;          // positions: one a thread, four threads a four-position block
+constexpr int A1_SCORES = 64 * 1024;   // positions * head size at most
+
+template <int HS> constexpr int a1_chunk() { return HS <= 64 ? HS : (HS % 64 == 0 ? 64 : 48); }  // dims in registers
+
+template <int HS, bool HALF>
+__global__ __launch_bounds__(A2_NT) void attend1_kernel(const AttnArgs a) {
+  constexpr int AC = A2_AC, S = HS / AC, DC = a1_chunk<HS>();
+  extern __shared__ float4 lds4[];
+  float *const lds = reinterpret_cast<float *>(lds4);
+  __shared__ float4 qs[HS / 4];
+  __shared__ float wave_mx[16], shared_inv;
+  const int mul = a.nh / a.nkv, groups = a.nkv * S;
+  const int xcd = blockIdx.x & 7, idx = blockIdx.x >> 3, hl = idx % mul, g = (idx / mul) * 8 + xcd;
+  if (g >= groups) return;  // the grid's rounding up: whole blocks leave
+  const int kh = g / S, j0 = (g % S) * AC, h = kh * mul + hl;
+  const int t = blockIdx.z, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int count = first_position(a) + t + 1, count4 = count & ~3, q4 = count4 >> 2, rs = chain_rowstride(q4);
+  float *const e4 = lds;             // [4][rs]
+  float *const tail = lds + 4 * rs;  // [4]
+  float *const blk = tail + 4;       // [AC][rs]
+  const int64_t vcol = (int64_t)(kh * HS + j0) * a.vstride;  // the block's first value column
+  const int kvdim = a.nkv * HS;
+  if (tid < HS / 4) qs[tid] = reinterpret_cast<const float4 *>(a.q + (int64_t)t * a.q_stride + (int64_t)h * HS)[tid];
+  // this thread's position's keys and its four-position block's values of 4 columns (clamped: never used past the count)
+  const int64_t krow = (int64_t)min(tid, count - 1) * kvdim + kh * HS;
+  const bool scoring = wave * 64 < count;  // uniform
+  float4 kr[DC / 4], v[4];
+  if (scoring) {
+#pragma unroll
+    for (int c = 0; c < DC / 4; ++c) kr[c] = cache4<HALF>(a.kcache, krow + 4 * c);
+  }
+  const int b = tid & 255, cg = tid >> 8, bc = max(min(b, q4 - 1), 0);
+#pragma unroll
+  for (int j = 0; j < 4; ++j) v[j] = cache4<HALF>(a.vcache, vcol + (int64_t)(4 * cg + j) * a.vstride + 4 * bc);
+  float tv[3];  // wave 0, lane j < AC: column j's values past the fours (at most 3)
+  if (wave == 0) {
+#pragma unroll
+    for (int r = 0; r < 3; ++r)
+      tv[r] = cache1<HALF>(a.vcache, vcol + (int64_t)(lane % AC) * a.vstride + min(count4 + r, count - 1));
+  }
+  lds_barrier();  // (the queries; the loads stay in flight)
+  float sc = -__builtin_inff();
+  if (scoring) {
+    float l0 = 0.0f, l1 = 0.0f, l2 = 0.0f, l3 = 0.0f;
+    for (int d = 0; d < HS; d += DC) {
+      if (d > 0) {
+#pragma unroll
+        for (int c = 0; c < DC / 4; ++c) kr[c] = cache4<HALF>(a.kcache, krow + d + 4 * c);
+      }
+#pragma unroll
+      for (int c = 0; c < DC / 4; ++c) {
+        const float4 qv = qs[d / 4 + c];
+        l0 = l0 + qv.x * kr[c].x;
+        l1 = l1 + qv.y * kr[c].y;
+        l2 = l2 + qv.z * kr[c].z;
+        l3 = l3 + qv.w * kr[c].w;
+      }
+    }
+    if (tid < count) sc = ((l0 + l2) + (l1 + l3)) * (1.0f / __builtin_sqrtf((float)HS));
+  }
+  float mx = sc;
+  for (int o = 32; o >= 1; o >>= 1) mx = wmax(mx, __shfl_xor(mx, o, 64));
+  if (lane == 0) wave_mx[wave] = mx;
+  lds_barrier();
+  mx = wave_mx[0];
+#pragma unroll
+  for (int w = 1; w < 16; ++w) mx = wmax(mx, wave_mx[w]);
+  if (tid < count) {
+    const float d = sc - mx;
+    if (tid < count4) e4[(tid & 3) * rs + (tid >> 2)] = vexp(d);
+    else tail[tid - count4] = fexp(d);
+  }
+  lds_barrier();
+  if (wave == 0) {
+    // lanes 0-3: lane k's sum; ((l0 + l1) + l2) + l3, the tail in order, 1 / sum
+    const float part = lane < 4 ? lds_chain_h<4>(e4 + lane * rs, q4, 0.0f) : 0.0f;
+    const float c1 = __shfl(part, 1, 64), c2 = __shfl(part, 2, 64), c3 = __shfl(part, 3, 64);
+    if (lane == 0) {
+      float sum = ((part + c1) + c2) + c3;
+      for (int r = 0; r < count - count4; ++r) sum = sum + tail[r];
+      shared_inv = 1.0f / sum;
+    }
+  }
+  lds_barrier();
+  const float inv = shared_inv;
+  if (b < q4) {
+    const float p0 = e4[b] * inv, p1 = e4[rs + b] * inv, p2 = e4[2 * rs + b] * inv, p3 = e4[3 * rs + b] * inv;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) blk[(4 * cg + j) * rs + b] = (p0 * v[j].x + p1 * v[j].y) + (p2 * v[j].z + p3 * v[j].w);
+  }
+  lds_barrier();
+  if (wave == 0 && lane < AC) {
+    float acc = lds_chain(blk + lane * rs, q4, 0.0f);
+#pragma unroll
+    for (int r = 0; r < 3; ++r)
+      if (r < count - count4) acc = acc + (tail[r] * inv) * tv[r];
+    a.out[(int64_t)t * a.out_stride + h * HS + j0 + lane] = acc;
+  }
+}
+
+// whether attend1_kernel takes a decode launch
+bool attend1_takes(const AttnArgs &a) {
+  const int count = a.pos0 + a.m;
+  return a.hs % A2_AC == 0 && count <= A1_MOST && count * a.hs <= A1_SCORES;
+}
+
 // LDS bytes of attend_kernel for the largest count of a launch (ring slots into *nslot), 0 where it does not fit
 template <int HS>
 int attend_lds(const AttnArgs &a, int *nslot) {
@@ -443,6 +557,12 @@ bool attend2_takes(const AttnArgs &a) {
 template <int HS, bool HALF>
 hipError_t launch_hs(const AttnArgs &a, hipStream_t s) {
   const int tiles = (a.pos0 + a.m + TILE - 1) / TILE;
+  if (a.m <= DECODE_TOKENS && !a.split && !a.xq && attend1_takes(a)) {
+    const int groups = a.nkv * (HS / A2_AC), g8 = (groups + 7) & ~7;
+    hipLaunchKernelGGL((attend1_kernel<HS, HALF>), dim3(g8 * (a.nh / a.nkv), 1, a.m), dim3(A2_NT),
+                       attend2_lds(a.pos0 + a.m), s, a);
+    return hipGetLastError();
+  }
   if (a.m <= DECODE_TOKENS) {
     hipLaunchKernelGGL((scores_kernel<HS, HALF>), dim3(tiles, a.nkv, a.m), dim3(256), 0, s, a);
   } else {

@@ -484,11 +484,10 @@ double matmul_bytes(const he_engine *e, const MatSeg *segs, int nseg, int32_t k,
   return b;
 }
 
-// the float32 source of a one-token matmul's activations, quantized in the launch (after rmsnorm with weights norm
-// where norm is not null): MatArgs.xf
+// the float32 source of a one-token matmul's activations, quantized in the launch: MatArgs.xf, x2, f32
 struct F32Source {
-  const float *x;
-  const float *norm;
+  int32_t kind;
+  const float *x, *x2;
 };
 
 hipError_t matmul_launch(he_engine *e, const MatSeg *segs, int nseg, int32_t k, int32_t m, const int8_t *xq,
@@ -507,8 +506,9 @@ hipError_t matmul_launch(he_engine *e, const MatSeg *segs, int nseg, int32_t k, 
   a.k = k;
   a.m = m;
   if (f32) {
+    a.f32 = f32->kind;
     a.xf = f32->x;
-    a.xnorm = f32->norm;
+    a.x2 = f32->x2;
     a.eps = e->c.rms_norm_eps;
   }
   if (qkv) a.qkv = *qkv;
@@ -576,8 +576,9 @@ hipError_t matmul(he_engine *e, const MatSeg *segs, int nseg, int32_t k, int32_t
                [&] { return matmul_launch(e, segs, nseg, k, m, xq, xs, f32, qkv, persistent); });
 }
 
-// one token whose rows of k the decode GEMV quantizes itself: it saves a launch where the GEMV is about one block a
-// CU (wo), and would cost more than it saves on the larger ones (each block repeats it). (Measured: rmsnorm in the
+// one token whose rows of k the decode GEMV quantizes itself (the attention's output, the FFN's activation): it saves a
+// launch where the GEMV is about one block a CU, and would cost more than it saves on the larger ones (each block repeats
+// it). (Measured: rmsnorm in the
 // q/k/v GEMV's blocks costs as much as its own launch, which is latency inside the norm, not the launch.)
 bool quantizes_itself(const he_engine *e, int32_t k, int32_t m, int32_t rows) {
   return m == 1 && rows <= 8192 && decode_takes_f32(k, e->c.six != 0, e->c.relaxed != 0);
@@ -675,7 +676,7 @@ int32_t run_chunk(he_engine *e, const int32_t *tokens, int32_t m, int32_t pos0, 
     // quantize_x in each block (an ordered sum of 256 steps at most), two launches a layer fewer. (At dim 4096 each
     // block repeating the 1024-step sum costs more than the launch.)
     const bool norm_in_gemv = !ln && m == 1 && dim <= 1024 && decode_takes_f32(dim, c.six != 0, c.relaxed != 0);
-    const F32Source att_src{e->x, e->vec(HE_T_RMS_ATT, (int64_t)l * dim)};
+    const F32Source att_src{F32_NORM, e->x, e->vec(HE_T_RMS_ATT, (int64_t)l * dim)};
     if (!ln && !norm_in_gemv) {
       const L2Fetch fq = fetch_for(e, qkv, 3, dim, m, 256, fuse_qkv);
       HIP_TRY(timed(e, HE_K_NORM, (double)m * dim * (8 + 1 + 0.125) + dim * 4.0, [&] {
@@ -747,7 +748,7 @@ int32_t run_chunk(he_engine *e, const int32_t *tokens, int32_t m, int32_t pos0, 
       HIP_TRY(matmul(e, wo, 1, qdim, m, e->xq, e->xs));
     } else if (wo_quantizes) {
       // the wide models' output projection on the persistent GEMV (each block quantizes the token once)
-      const F32Source src{e->xb, nullptr};
+      const F32Source src{F32_RAW, e->xb, nullptr};
       HIP_TRY(matmul(e, wo, 1, qdim, m, e->xq, e->xs, &src, nullptr, true));
     } else {
       HIP_TRY(timed(e, HE_K_NORM, (double)m * qdim * (4 + 1 + 0.125),
@@ -771,6 +772,11 @@ int32_t run_chunk(he_engine *e, const int32_t *tokens, int32_t m, int32_t pos0, 
       }
       const MatSeg w1[1] = {{e->mat(HE_T_W1, l), e->mat_scales(HE_T_W1, l), e->hb, hidden, hidden, 0}};
       HIP_TRY(matmul(e, w1, 1, dim, m, e->xq, e->xs));
+      if (quantizes_itself(e, hidden, m, dim)) {
+        const F32Source src{F32_GELU, e->hb, b1};
+        HIP_TRY(matmul(e, w2, 1, hidden, m, e->xq, e->xs, &src));
+        continue;
+      }
       HIP_TRY(timed(e, HE_K_ELEMENTWISE, (double)m * hidden * (8 + 1 + 0.125), [&] {
         return launch_gelu_quant(e->xq, e->xs, nullptr, e->hb, b1, m, hidden, hidden, W, W / 32, e->bias, s);
       }));
@@ -792,8 +798,13 @@ int32_t run_chunk(he_engine *e, const int32_t *tokens, int32_t m, int32_t pos0, 
       HIP_TRY(matmul(e, w2, 1, hidden, m, gq, e->hb2));
       continue;
     }
-    const F32Source ffn_src{e->x, e->vec(HE_T_RMS_FFN, (int64_t)l * dim)};
+    const F32Source ffn_src{F32_NORM, e->x, e->vec(HE_T_RMS_FFN, (int64_t)l * dim)};
     HIP_TRY(matmul(e, w13, 2, dim, m, e->xq, e->xs, norm_in_gemv ? &ffn_src : nullptr));
+    if (quantizes_itself(e, hidden, m, dim)) {
+      const F32Source src{F32_SWIGLU, e->hb, e->hb2};
+      HIP_TRY(matmul(e, w2, 1, hidden, m, e->xq, e->xs, &src));
+      continue;
+    }
     HIP_TRY(timed(e, HE_K_ELEMENTWISE, (double)m * hidden * (8 + 1 + 0.125), [&] {
       return launch_swiglu_quant(e->xq, e->xs, nullptr, e->hb, e->hb2, m, hidden, hidden, W, W / 32, e->bias, s);
     }));

@@ -250,8 +250,9 @@ __global__ __launch_bounds__(256) void gemv_kernel(const MatArgs a) {
   }
 }
 
-// The activations of a decode launch from the float32 token instead of quantize_x's output, in the block itself (no
-// launch of their own): with a.xnorm, rmsnorm first (kernels/kernel.ts:330-342: the squares in four lanes j % 4 added
+// The activations of a decode launch from float32 values instead of quantize_x's output, in the block itself (no
+// launch of their own): for F32_SWIGLU and F32_GELU the FFN's activation first (misc.hip swiglu_quant_kernel, forms.hip
+// gelu_quant_kernel), for F32_NORM rmsnorm (kernels/kernel.ts:330-342: the squares in four lanes j % 4 added
 // in order by four threads, hsum ((l0 + l1) + l2) + l3, the tail; s = f32(1 / f32(sqrt(f32(ss / n) + eps)));
 // out = w * (s * x)), then quantize_x with bias 64 (kernels/kernel.ts:129-156), stored centred (q - 64) into xl with the
 // group scales into xsl. Every block computes the same bits. Thread tid of the block's NT takes the MAXU consecutive
@@ -259,9 +260,9 @@ __global__ __launch_bounds__(256) void gemv_kernel(const MatArgs a) {
 // the rows as float4; a group of 32 is then 32 / MAXU neighbouring lanes, whose largest magnitude is their own
 // maxima's (DPP within the group's lanes), so that a lane computes one group's scale and its reciprocal, not MAXU of
 // them. sq: 4 * chain_rowstride(K / 4) floats of LDS.
-// NORM (rmsnorm with a.xnorm) is a template argument: a load under a run-time test of the pointer is waited for
+// SRC (a.f32) is a template argument: a load under a run-time test of the pointer is waited for
 // before the next is requested, which made the token's loads one round trip each.
-template <int MAXU, bool NORM, int NT = 256>
+template <int MAXU, int SRC, int NT = 256>
 __device__ __forceinline__ void load_f32(const MatArgs &a, float (&xv)[MAXU], float (&wv)[MAXU]) {
   static_assert(MAXU % 4 == 0 && 32 % MAXU == 0, "a lane's positions: whole float4, within one group");
 #pragma unroll
@@ -269,8 +270,8 @@ __device__ __forceinline__ void load_f32(const MatArgs &a, float (&xv)[MAXU], fl
     const int j = min((int)threadIdx.x * MAXU + 4 * u, a.k - 4);  // clamped: every load unconditional
     const float4 x4 = *reinterpret_cast<const float4 *>(a.xf + j);
     xv[4 * u] = x4.x; xv[4 * u + 1] = x4.y; xv[4 * u + 2] = x4.z; xv[4 * u + 3] = x4.w;
-    if constexpr (NORM) {
-      const float4 w4 = *reinterpret_cast<const float4 *>(a.xnorm + j);
+    if constexpr (SRC != F32_RAW) {
+      const float4 w4 = *reinterpret_cast<const float4 *>(a.x2 + j);
       wv[4 * u] = w4.x; wv[4 * u + 1] = w4.y; wv[4 * u + 2] = w4.z; wv[4 * u + 3] = w4.w;
     } else {
 #pragma unroll
@@ -278,14 +279,14 @@ __device__ __forceinline__ void load_f32(const MatArgs &a, float (&xv)[MAXU], fl
     }
   }
 }
-template <int MAXU, bool NORM, int NT = 256>
+template <int MAXU, int SRC, int NT = 256>
 __device__ __forceinline__ void stage_from_f32(const MatArgs &a, const float (&xv)[MAXU], const float (&wv)[MAXU],
                                                uint8_t *xl, float *xsl, float *sq) {
   __shared__ float part[4], sval;
   constexpr int LG = 32 / MAXU;  // lanes a group
   const int tid = threadIdx.x, K = a.k, q4 = K >> 2, qs = chain_rowstride(q4), j0 = tid * MAXU;
   float sc = 1.0f;
-  if constexpr (NORM) {
+  if constexpr (SRC == F32_NORM) {
     if (j0 < K) {
 #pragma unroll
       for (int i = 0; i < MAXU; ++i) sq[(i & 3) * qs + ((j0 + i) >> 2)] = xv[i] * xv[i];
@@ -301,7 +302,16 @@ __device__ __forceinline__ void stage_from_f32(const MatArgs &a, const float (&x
   float m = 0.0f;
 #pragma unroll
   for (int i = 0; i < MAXU; ++i) {
-    o[i] = NORM ? wv[i] * (sc * xv[i]) : xv[i];
+    if constexpr (SRC == F32_NORM) {
+      o[i] = wv[i] * (sc * xv[i]);
+    } else if constexpr (SRC == F32_SWIGLU) {
+      o[i] = xv[i] / (1.0f + vexp(-xv[i])) * wv[i];
+    } else if constexpr (SRC == F32_GELU) {
+      const float h = xv[i] + wv[i], inner = 0.7978845608028654f * (h + ((0.044715f * h) * h) * h);
+      o[i] = h / (1.0f + vexp(-2.0f * inner));
+    } else {
+      o[i] = xv[i];
+    }
     m = __builtin_fmaxf(m, __builtin_fabsf(o[i]));
   }
   // the group's largest magnitude (order-free): xor 1 and xor 2 within quads, then the mirror within 8 lanes
@@ -330,7 +340,7 @@ __device__ __forceinline__ void stage_from_f32(const MatArgs &a, const float (&x
 // the loads next to their uses); meanwhile the block stages the token's activations, centred, and their scales in
 // LDS once. The R rows' products go to LDS and 4R lanes add them in the reference's order at once.
 // NS: wave steps (1 KiB of a row), NS * 1024 >= K.
-// SRC: 0 the activations from xq / xs; 1 the float32 token (a.xf); 2 a.xf after rmsnorm with a.xnorm
+// SRC: the activations from xq / xs (F32_NONE), or what a.f32 says
 template <int R, int NS, int SRC>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 4))) void gemv1_kernel(const MatArgs a) {
   constexpr bool F32 = SRC != 0;
@@ -358,7 +368,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 4))) voi
   float fx[FU], fw[FU];
   if constexpr (F32) {
     static_assert(NS <= 4, "the float32 token is held a thread at a time");
-    load_f32<FU, SRC == 2>(a, fx, fw);
+    load_f32<FU, SRC>(a, fx, fw);
   } else {
 #pragma unroll
     for (int u = 0; u < XL; ++u) xv[u] = reinterpret_cast<const uint4 *>(a.xq)[min((int)threadIdx.x + 256 * u, K / 16 - 1)];
@@ -397,7 +407,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 4))) voi
   __builtin_amdgcn_sched_barrier(0);
   // the block's activations into LDS: K / 16 uint4, centred (or made here from the float32 token)
   if constexpr (F32) {
-    stage_from_f32<FU, SRC == 2>(a, fx, fw, reinterpret_cast<uint8_t *>(xl), xsl, P - wave * R * lay.stride);
+    stage_from_f32<FU, SRC>(a, fx, fw, reinterpret_cast<uint8_t *>(xl), xsl, P - wave * R * lay.stride);
   } else {
 #pragma unroll
     for (int u = 0; u < XL; ++u) {
@@ -464,9 +474,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 4))) voi
 // of block b takes the row groups gw, gw + NWV, gw + 2 NWV, ... (gw = b PW + w, NWV = every wave of the grid) of R
 // consecutive rows, requesting a group's rows and scales, then adding them up, then the next group. The CU hides each
 // wave's load latency behind its other waves' groups. The block stages the token's activations in LDS once, while
-// every wave's first group is in flight: from xq / xs (centred), or (F32) from the float32 token, after rmsnorm where
-// a.xnorm is given, in the block itself (stage_from_f32), so that the norm's ordered sum runs once a CU while HBM
-// delivers the first rows, instead of in a launch of its own. Per row the arithmetic is gemv1_kernel's: exact group
+// every wave's first group is in flight: from xq / xs (centred), or (F32) from the float32 token in the block itself
+// (stage_from_f32). Per row the arithmetic is gemv1_kernel's: exact group
 // sums by v_dot4, their float32 products into LDS, 4R lanes adding the reference's four chains in order, and
 // store_row (the residual add, or the q / k / v epilogue).
 template <int R, int NS>
@@ -596,7 +605,7 @@ __device__ __forceinline__ void finish_rows(const RowSet<R, NS> &b, const MatArg
   wave_sync_lds();  // the next group writes wsl and P again
 }
 
-// SRC: 0 the activations from xq / xs; 1 the float32 token (a.xf); 2 a.xf after rmsnorm with a.xnorm
+// SRC: the activations from xq / xs (F32_NONE), or the float32 token (F32_RAW)
 template <int PW, int R, int NS, int SRC, bool ALIGNED>
 __global__ __launch_bounds__(64 * PW) void gemvp_kernel(const MatArgs a) {
   constexpr int PNT = 64 * PW;
@@ -611,7 +620,6 @@ __global__ __launch_bounds__(64 * PW) void gemvp_kernel(const MatArgs a) {
   float *xsl = smem + K / 4;                                       // G scales of the activations
   float *wsl = xsl + G16 + wave * R * G16;                         // this wave's rows' weight scales
   float *P = xsl + G16 + PW * R * G16 + wave * R * lay.stride;     // this wave's products
-  float *sq = xsl + G16 + PW * R * G16 + PW * R * lay.stride;      // F32 with a norm: the squares' four rows
   const int ngroups = (a.total_rows + R - 1) / R, nwv = gridDim.x * PW;
   int group = blockIdx.x * PW + wave;
   const SegPick sp = seg_pick(a);
@@ -624,7 +632,7 @@ __global__ __launch_bounds__(64 * PW) void gemvp_kernel(const MatArgs a) {
   float sv[XSV];
   float fx[FU], fw[FU];
   if constexpr (F32) {
-    load_f32<FU, SRC == 2, PNT>(a, fx, fw);
+    load_f32<FU, SRC, PNT>(a, fx, fw);
   } else {
 #pragma unroll
     for (int u = 0; u < XL; ++u) xv[u] = reinterpret_cast<const uint4 *>(a.xq)[min((int)threadIdx.x + PNT * u, K / 16 - 1)];
@@ -634,7 +642,7 @@ __global__ __launch_bounds__(64 * PW) void gemvp_kernel(const MatArgs a) {
   request_rows<R, NS, ALIGNED>(rows, sp, K, a.total_rows, group, ngroups, lane);
   __builtin_amdgcn_sched_barrier(0);
   if constexpr (F32) {
-    stage_from_f32<FU, SRC == 2, PNT>(a, fx, fw, reinterpret_cast<uint8_t *>(xl), xsl, sq);
+    stage_from_f32<FU, SRC, PNT>(a, fx, fw, reinterpret_cast<uint8_t *>(xl), xsl, nullptr);
   } else {
 #pragma unroll
     for (int u = 0; u < XL; ++u) {
@@ -662,7 +670,7 @@ __global__ __launch_bounds__(64 * PW) void gemvp_kernel(const MatArgs a) {
 // gemv1_kernel, with a lane taking two consecutive groups of 24 bytes (48 bytes, three 16-byte loads) of each of its
 // wave's R rows, 128 groups a wave step, widened to int8 in registers (kernels/six.ts) next to their use.
 // NS: wave steps, NS * 128 groups >= K / 32.
-// SRC: 0 the activations from xq / xs; 1 the float32 token (a.xf); 2 a.xf after rmsnorm with a.xnorm
+// SRC: the activations from xq / xs (F32_NONE), or what a.f32 says
 // W: waves a block (the float32 token's blocks take 16, so that quantize_x of the token is 4 values a thread)
 template <int R, int NS, int SRC, int W>
 __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(1, 4))) void gemv6_kernel(const MatArgs a) {
@@ -690,7 +698,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(1, 4))) 
   float fx[FU], fw[FU];
   if constexpr (F32) {
     static_assert(NS == 1, "the float32 token is held a thread at a time");
-    load_f32<FU, SRC == 2, NT>(a, fx, fw);
+    load_f32<FU, SRC, NT>(a, fx, fw);
   } else {
 #pragma unroll
     for (int u = 0; u < XL; ++u) xv[u] = reinterpret_cast<const uint4 *>(a.xq)[min((int)threadIdx.x + NT * u, K / 16 - 1)];
@@ -728,7 +736,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(1, 4))) 
     }
   __builtin_amdgcn_sched_barrier(0);
   if constexpr (F32) {
-    stage_from_f32<FU, SRC == 2, NT>(a, fx, fw, reinterpret_cast<uint8_t *>(xl), xsl, P - wave * R * lay.stride);
+    stage_from_f32<FU, SRC, NT>(a, fx, fw, reinterpret_cast<uint8_t *>(xl), xsl, P - wave * R * lay.stride);
   } else {
 #pragma unroll
     for (int u = 0; u < XL; ++u) {
@@ -809,16 +817,18 @@ hipError_t launch_gemv6(const MatArgs &a, hipStream_t s) {
   const size_t g16 = ((a.k / GS) + 3) & ~3;
   const size_t head = (size_t)a.k + sizeof(float) * g16 * (1 + W * R);
   size_t products = sizeof(float) * W * R * (size_t)row_layout(a.k, true).stride;
-  if (a.xf) products = std::max(products, sizeof(float) * 4 * (size_t)chain_rowstride(a.k / 4));  // the squares
+  if (a.f32 == F32_NORM) products = std::max(products, sizeof(float) * 4 * (size_t)chain_rowstride(a.k / 4));  // squares
   const size_t lds = head + products;
   if constexpr (NS == 1) {
-    if (a.xf) {
-      if (a.xnorm) hipLaunchKernelGGL((gemv6_kernel<R, NS, 2, W>), dim3(blocks), dim3(64 * W), lds, s, a);
-      else hipLaunchKernelGGL((gemv6_kernel<R, NS, 1, W>), dim3(blocks), dim3(64 * W), lds, s, a);
-      return hipGetLastError();
+    switch (a.f32) {
+      case F32_RAW: hipLaunchKernelGGL((gemv6_kernel<R, NS, F32_RAW, W>), dim3(blocks), dim3(64 * W), lds, s, a); break;
+      case F32_NORM: hipLaunchKernelGGL((gemv6_kernel<R, NS, F32_NORM, W>), dim3(blocks), dim3(64 * W), lds, s, a); break;
+      case F32_SWIGLU: hipLaunchKernelGGL((gemv6_kernel<R, NS, F32_SWIGLU, W>), dim3(blocks), dim3(64 * W), lds, s, a); break;
+      case F32_GELU: hipLaunchKernelGGL((gemv6_kernel<R, NS, F32_GELU, W>), dim3(blocks), dim3(64 * W), lds, s, a); break;
     }
+    if (a.xf) return hipGetLastError();
   }
-  hipLaunchKernelGGL((gemv6_kernel<R, NS, 0, W>), dim3(blocks), dim3(64 * W), lds, s, a);
+  hipLaunchKernelGGL((gemv6_kernel<R, NS, F32_NONE, W>), dim3(blocks), dim3(64 * W), lds, s, a);
   return hipGetLastError();
 }
 
@@ -850,16 +860,18 @@ hipError_t launch_gemv1(const MatArgs &a, hipStream_t s) {
   const size_t g16 = ((a.k / GS) + 3) & ~3;
   const size_t head = (size_t)a.k + sizeof(float) * g16 * (1 + WAVES * R);
   size_t products = sizeof(float) * WAVES * R * (size_t)row_layout(a.k, true).stride;
-  if (a.xf) products = std::max(products, sizeof(float) * 4 * (size_t)chain_rowstride(a.k / 4));  // the squares
+  if (a.f32 == F32_NORM) products = std::max(products, sizeof(float) * 4 * (size_t)chain_rowstride(a.k / 4));  // squares
   const size_t lds = head + products;
   if constexpr (NS <= 4) {
-    if (a.xf) {
-      if (a.xnorm) hipLaunchKernelGGL((gemv1_kernel<R, NS, 2>), dim3(blocks), dim3(64 * WAVES), lds, s, a);
-      else hipLaunchKernelGGL((gemv1_kernel<R, NS, 1>), dim3(blocks), dim3(64 * WAVES), lds, s, a);
-      return hipGetLastError();
+    switch (a.f32) {
+      case F32_RAW: hipLaunchKernelGGL((gemv1_kernel<R, NS, F32_RAW>), dim3(blocks), dim3(64 * WAVES), lds, s, a); break;
+      case F32_NORM: hipLaunchKernelGGL((gemv1_kernel<R, NS, F32_NORM>), dim3(blocks), dim3(64 * WAVES), lds, s, a); break;
+      case F32_SWIGLU: hipLaunchKernelGGL((gemv1_kernel<R, NS, F32_SWIGLU>), dim3(blocks), dim3(64 * WAVES), lds, s, a); break;
+      case F32_GELU: hipLaunchKernelGGL((gemv1_kernel<R, NS, F32_GELU>), dim3(blocks), dim3(64 * WAVES), lds, s, a); break;
     }
+    if (a.xf) return hipGetLastError();
   }
-  hipLaunchKernelGGL((gemv1_kernel<R, NS, 0>), dim3(blocks), dim3(64 * WAVES), lds, s, a);
+  hipLaunchKernelGGL((gemv1_kernel<R, NS, F32_NONE>), dim3(blocks), dim3(64 * WAVES), lds, s, a);
   return hipGetLastError();
 }
 
@@ -879,13 +891,11 @@ int persistent_blocks() {
 
 constexpr size_t PLDS = 160 * 1024 - 1024;  // LDS a persistent block may take (gfx950: 160 KiB a workgroup)
 
-// the LDS of a persistent block: the activations and their scales, every wave's rows' scales and products, the squares
-size_t gemvp_lds(int pw, int r, int k, bool norm) {
+// the LDS of a persistent block: the activations and their scales, every wave's rows' scales and products
+size_t gemvp_lds(int pw, int r, int k) {
   const size_t g16 = ((k / GS) + 3) & ~3;
-  size_t lds = (size_t)k + sizeof(float) * g16 * (1 + (size_t)pw * r) +
-               sizeof(float) * (size_t)pw * r * (size_t)row_layout(k, true).stride;
-  if (norm) lds += sizeof(float) * 4 * (size_t)chain_rowstride(k / 4);
-  return lds;
+  return (size_t)k + sizeof(float) * g16 * (1 + (size_t)pw * r) +
+         sizeof(float) * (size_t)pw * r * (size_t)row_layout(k, true).stride;
 }
 
 template <int PW, int R, int NS, int SRC, bool ALIGNED>
@@ -910,21 +920,18 @@ hipError_t launch_gemvp(const MatArgs &a, hipStream_t s, int blocks_a_cu = 1) {
   if (f32 && (NS > 4 || a.k % 32)) return hipErrorInvalidValue;
   const int G = a.k / GS, ngroups = (a.total_rows + R - 1) / R;
   const int blocks = std::min((ngroups + PW - 1) / PW, blocks_a_cu * persistent_blocks());
-  const size_t lds = gemvp_lds(PW, R, a.k, f32 && a.xnorm);
+  const size_t lds = gemvp_lds(PW, R, a.k);
   if (lds > PLDS) return hipErrorInvalidValue;
   // the rows' scales as float4 where every segment's start and row length keep them on 16 bytes
   bool aligned = G % 4 == 0;
   for (int i = 0; i < a.nseg; ++i) aligned = aligned && reinterpret_cast<uintptr_t>(a.seg[i].ws) % 16 == 0;
   if constexpr (NS <= 4) {
-    if (f32 && a.xnorm)
-      return aligned ? launch_gemvp_one<PW, R, NS, 2, true>(a, blocks, lds, s)
-                     : launch_gemvp_one<PW, R, NS, 2, false>(a, blocks, lds, s);
     if (f32)
-      return aligned ? launch_gemvp_one<PW, R, NS, 1, true>(a, blocks, lds, s)
-                     : launch_gemvp_one<PW, R, NS, 1, false>(a, blocks, lds, s);
+      return aligned ? launch_gemvp_one<PW, R, NS, F32_RAW, true>(a, blocks, lds, s)
+                     : launch_gemvp_one<PW, R, NS, F32_RAW, false>(a, blocks, lds, s);
   }
-  return aligned ? launch_gemvp_one<PW, R, NS, 0, true>(a, blocks, lds, s)
-                 : launch_gemvp_one<PW, R, NS, 0, false>(a, blocks, lds, s);
+  return aligned ? launch_gemvp_one<PW, R, NS, F32_NONE, true>(a, blocks, lds, s)
+                 : launch_gemvp_one<PW, R, NS, F32_NONE, false>(a, blocks, lds, s);
 }
 
 // the persistent path (measured on the 8B shapes: 8 waves a block and 2 rows a group for rows of 2-4 KiB, the output
@@ -1029,6 +1036,8 @@ hipError_t launch_gemv(const MatArgs &a, bool six, bool relaxed, hipStream_t s) 
   const bool sums = a.sums != nullptr;
   if (a.xf && (sums || a.m != 1 || !decode_takes_f32(a.k, six, relaxed))) return hipErrorInvalidValue;
   if (a.qkv.on && (sums || a.m != 1 || !decode_fuses_qkv(a.k, six, relaxed))) return hipErrorInvalidValue;
+  if ((a.f32 != F32_NONE) != (a.xf != nullptr) || (a.f32 > F32_RAW && !a.x2)) return hipErrorInvalidValue;
+  if (a.persistent && a.f32 > F32_RAW) return hipErrorInvalidValue;
   if (a.persistent && (sums || a.m != 1 || !decode_persistent(a.k, six, relaxed))) return hipErrorInvalidValue;
   if (a.persistent) return launch_persistent(a, s);
   if (!sums && !six && relaxed && a.m == 1 && a.k <= 20 * 1024) return launch_decode(a, s);

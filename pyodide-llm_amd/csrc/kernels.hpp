@@ -61,6 +61,7 @@ struct GluOut {
   float *s;   // [m][s_stride]
   int32_t q_stride, s_stride, bias;
 };
+enum { F32_NONE = 0, F32_RAW, F32_NORM, F32_SWIGLU, F32_GELU };
 struct MatArgs {
   MatSeg seg[3];
   int32_t nseg;
@@ -72,11 +73,13 @@ struct MatArgs {
   int32_t k;
   int32_t m;
   int32_t *sums;  // group-sum output (hk_group_sums) or null
-  // one token (the decode path, decode_takes_f32): the float32 token instead of xq / xs, quantized in the launch,
-  // after rmsnorm with weights xnorm (and eps) where xnorm is not null
+  // one token (the decode path, decode_takes_f32): float32 values instead of xq / xs, quantized in the launch after what
+  // f32 says: as they are, after rmsnorm with the weights x2 (and eps), as h1 of the SwiGLU with h3 x2, or after
+  // gelu(xf + x2)
   const float *xf;
-  const float *xnorm;
+  const float *x2;
   float eps;
+  int32_t f32;
   QkvFuse qkv;  // decode_fuses_qkv()
   // one token, rows of 1-4 KiB (decode_persistent): the persistent GEMV, about one block a CU that loops over its
   // rows (no L2Fetch fits it: its blocks take rows in another order)
