@@ -15,19 +15,18 @@ namespace ple {
 
 // i32.trunc_sat_f32_s: NaN to 0, out of range to the nearest end (the conversion of quantize_x, kernels/kernel.ts:145)
 // (as selects: the clamped conversion, then the top end and NaN)
+// (the conversion instruction's own results)
 __device__ __forceinline__ int32_t trunc_sat(float f) {
-  const float c = __builtin_fminf(__builtin_fmaxf(f, -2147483648.0f), 2147483520.0f);
-  int32_t r = (int32_t)c;
-  r = f >= 2147483648.0f ? 2147483647 : r;
-  return __builtin_isnan(f) ? 0 : r;
+  int32_t i;
+  asm("v_cvt_i32_f32 %0, %1" : "=v"(i) : "v"(f));
+  return i;
 }
-__device__ __forceinline__ int32_t sat16(int32_t v) { return v > 32767 ? 32767 : (v < -32768 ? -32768 : v); }
 __device__ __forceinline__ int32_t sat8(int32_t v) { return v > 127 ? 127 : (v < -128 ? -128 : v); }
 
 // quantize_x's value: narrow(trunc_sat(nearest(x * inv)) + bias) (kernels/kernel.ts:145-153; the i32 add wraps)
 __device__ __forceinline__ int8_t quant_value(float x, float inv, int32_t bias) {
   const int32_t t = (int32_t)((uint32_t)trunc_sat(__builtin_rintf(x * inv)) + (uint32_t)bias);
-  return (int8_t)sat8(sat16(t));
+  return (int8_t)sat8(t);  // (i16x8.narrow before i8x16.narrow changes nothing)
 }
 
 // four activations of quantize_x(bias 64) with the bias taken out, q - 64 per byte: (q + 0x40) ^ 0x80 for q in
@@ -56,24 +55,17 @@ __device__ __forceinline__ void six_widen(const uint32_t L[4], uint32_t T0, uint
 
 __device__ __forceinline__ float bits_f32(uint32_t u) { return __uint_as_float(u); }
 
-// f32x4.max / f32x4.min of WebAssembly: NaN if either is, else the larger / smaller (+0 above -0); written as
-// selects, so that no branch splits a wave
-__device__ __forceinline__ float wmax(float a, float b) {
-  const float larger = a > b ? a : b;
-  const float equal = __builtin_signbitf(a) ? b : a;
-  const float r = a == b ? equal : larger;
-  return __builtin_isunordered(a, b) ? a + b : r;
-}
-__device__ __forceinline__ float wmin(float a, float b) {
-  const float smaller = a < b ? a : b;
-  const float equal = __builtin_signbitf(a) ? a : b;
-  const float r = a == b ? equal : smaller;
-  return __builtin_isunordered(a, b) ? a + b : r;
-}
+// f32x4.max / f32x4.min of WebAssembly: NaN if either is, else the larger / smaller (+0 above -0): IEEE 754-2019's maximum
+// and minimum, one instruction each
+__device__ __forceinline__ float wmax(float a, float b) { return __builtin_elementwise_maximum(a, b); }
+__device__ __forceinline__ float wmin(float a, float b) { return __builtin_elementwise_minimum(a, b); }
 
 // the Cephes expf polynomial (S. L. Moshier's Cephes library) in the steps of kernels/kernel.ts:18-28
+// (x in [-87, 88] or NaN. The nearest integer k by adding 1.5 * 2^23, whose sum's low bits are k, so that 2^k is those bits
+// shifted: 28 VALU instructions a vexp with its two clamps, 42 with rint, a conversion and compares. The same bits for
+// every float32.)
 __device__ __forceinline__ float cephes_core(float x) {
-  const float k = __builtin_rintf(x * 1.44269504088896341f);
+  const float m = x * 1.44269504088896341f + 12582912.0f, k = m - 12582912.0f;
   const float r = (x - k * 0.693359375f) - k * -2.12194440e-4f;
   float p = 1.9875691500e-4f;
   p = p * r + 1.3981999507e-3f;
@@ -82,7 +74,7 @@ __device__ __forceinline__ float cephes_core(float x) {
   p = p * r + 1.6666665459e-1f;
   p = p * r + 5.0000001201e-1f;
   const float e = (p * (r * r) + r) + 1.0f;
-  return e * bits_f32((uint32_t)(trunc_sat(k) + 127) << 23);
+  return e * bits_f32((__float_as_uint(m) << 23) + (127u << 23));
 }
 // kernels/kernel.ts:15-29 fexp: 0 below -87, 88 above 88
 __device__ __forceinline__ float fexp(float x) {
