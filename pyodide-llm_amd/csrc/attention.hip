@@ -113,6 +113,22 @@ __device__ __forceinline__ void wait_at_least(const int *p, int v) {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
 }
 
+// +0.0 from the end of `rows` sums' rows of q4 values to the end of their last segment (chain16_registers), by the block's
+// first 32 * rows threads
+__device__ __forceinline__ void pad_rows(float *c, int rows, int rs, int q4, int tid) {
+  const int row = tid >> 5, i = (q4 & ~31) + (tid & 31);
+  if (row < rows && i >= q4 && (q4 & 31)) c[row * rs + chain16_at(i)] = 0.0f;
+}
+
+// 1 / the exponentials' sum: the four lanes' sums, ((l0 + l1) + l2) + l3, the tail in order; one wave, the same in each lane
+__device__ __forceinline__ float inverse_sum(const float *e4, int rs, int q4, const float *tail, int rest, int lane) {
+  const float part = chain16_registers<false>(e4 + (lane >> 4) * rs, q4, lane & 15);
+  float sum = ((chain16_result(part, q4, 0) + chain16_result(part, q4, 1)) + chain16_result(part, q4, 2)) +
+              chain16_result(part, q4, 3);
+  for (int r = 0; r < rest; ++r) sum = sum + tail[r];
+  return 1.0f / sum;
+}
+
 // an item's values: lane = four-position block, one float4 of positions a column of the item's 16 (clamped: never
 // added past count4)
 #define ATT_FETCH(item, v)                                                                                    \
@@ -186,22 +202,17 @@ __global__ __launch_bounds__(Attend<HS>::NT) void attend_kernel(const AttnArgs a
         const int i = base + tid + NT * u;
         if (i < count) {
           const float d = sv[u] - mx;
-          if (i < count4) e4[(i & 3) * rs + (i >> 2)] = vexp(d);
+          if (i < count4) e4[(i & 3) * rs + chain16_at(i >> 2)] = vexp(d);
           else tail[i - count4] = fexp(d);
         }
       }
     }
   }
+  pad_rows(e4, 4, rs, q4, tid);
   __syncthreads();
   if (wave == 0) {
-    // lanes 0-3: lane k's sum; ((l0 + l1) + l2) + l3, the tail in order, 1 / sum
-    const float part = lane < 4 ? lds_chain(e4 + lane * rs, q4, 0.0f) : 0.0f;
-    const float c1 = __shfl(part, 1, 64), c2 = __shfl(part, 2, 64), c3 = __shfl(part, 3, 64);
-    if (lane == 0) {
-      float sum = ((part + c1) + c2) + c3;
-      for (int r = 0; r < count - count4; ++r) sum = sum + tail[r];
-      shared_inv = 1.0f / sum;
-    }
+    const float inv = inverse_sum(e4, rs, q4, tail, count - count4, lane);
+    if (lane == 0) shared_inv = inv;
   }
   __syncthreads();
   const float inv = shared_inv;
@@ -210,7 +221,8 @@ __global__ __launch_bounds__(Attend<HS>::NT) void attend_kernel(const AttnArgs a
       const int c = it / H, half = it % H;
       wait_at_least(&used, c - nslot + 1);  // the slot's last chunk has been added
       float *slot = ring + (c % nslot) * (AC * RR) + half * 16 * RR + lane;
-      const int b = min(c * RB + lane, q4 - 1);  // the lane's four-position block (clamped: never added past q4)
+      // the lane's four-position block (clamped: never added past q4)
+      const int b = chain16_at(min(c * RB + lane, q4 - 1));
       const float p0 = e4[b] * inv, p1 = e4[rs + b] * inv, p2 = e4[2 * rs + b] * inv, p3 = e4[3 * rs + b] * inv;
 #pragma unroll
       for (int j = 0; j < 16; ++j) {
@@ -295,12 +307,13 @@ __global__ __launch_bounds__(Attend<HS>::NT) void attend_kernel(const AttnArgs a
 // (B + C) for a few tokens (decode) whose output the caller quantizes itself: one block of 1024 threads a (token,
 // query head, 16 columns), thread b owning the four-position block b (positions 4b .. 4b+3) of the weighted values.
 // The head's tile maxima and scores are requested at once, the exponentials go into LDS by lane (four rows: positions
-// t % 4 == k); then every thread requests its block's 16 columns x 4 values while four lanes of wave 0 run the
-// ordered sums, turns them into the columns' four-position products ((p0 v0 + p1 v1) + (p2 v2 + p3 v3)), p = e *
-// f32(1 / sum), into LDS rows (one a column), and 16 lanes of wave 0 add their column's products in order, then the
-// tail. (The values are requested once the exponentials are in LDS: requested at the start, their arrival slowed the
-// scores' loads and the exponentials.) Blocks of the query heads that share a kv head's columns go to one XCD, as in
-// attend_kernel.
+// t % 4 == k); then every thread requests its block's 16 columns x 4 values while wave 0 runs the ordered sums, turns
+// them into the columns' four-position products ((p0 v0 + p1 v1) + (p2 v2 + p3 v3)), p = e * f32(1 / sum), into LDS
+// rows (one a column), and waves 0-3 add the columns' products in order, a column a row of 16 lanes, then the tail.
+// (The values are requested once the exponentials are in LDS: requested at the start, their arrival slowed the scores'
+// loads and the exponentials.) The sums from registers (chain16_registers) instead of four and sixteen lanes' LDS reads:
+// 2060 positions, 32 / 8 heads of 128, scores included, 13.7 -> 12.8 us; 7002 positions 28.3 -> 26.1. Blocks of the query
+// heads that share a kv head's columns go to one XCD, as in attend_kernel.
 constexpr int A2_NT = 1024;  // threads a block
 constexpr int A2_AC = 16;    // columns a block
 constexpr int A2_SV = 4;     // scores a thread a pass (4096 positions)
@@ -314,16 +327,14 @@ size_t attend2_lds(int count) {
 }
 
 template <int HS, bool HALF>
-__global__ __launch_bounds__(A2_NT) void attend2_kernel(const AttnArgs a) {
+__device__ __forceinline__ void attend2(const AttnArgs &a, float *const lds) {
   constexpr int NT = A2_NT, AC = A2_AC, S = HS / AC;
-  extern __shared__ float4 lds4[];
-  float *const lds = reinterpret_cast<float *>(lds4);
   __shared__ float shared_mx, shared_inv;
   const int mul = a.nh / a.nkv, groups = a.nkv * S;
   const int xcd = blockIdx.x & 7, idx = blockIdx.x >> 3, hl = idx % mul, g = (idx / mul) * 8 + xcd;
   if (g >= groups) return;  // the grid's rounding up: whole blocks leave
   const int kh = g / S, j0 = (g % S) * AC, h = kh * mul + hl;
-  const int t = blockIdx.z, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int t = blockIdx.z, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int count = first_position(a) + t + 1, count4 = count & ~3, q4 = count4 >> 2, rs = chain_rowstride(q4);
   float *const e4 = lds;             // [4][rs]
   float *const tail = lds + 4 * rs;  // [4]
@@ -340,11 +351,13 @@ __global__ __launch_bounds__(A2_NT) void attend2_kernel(const AttnArgs a) {
   float sv[A2_SV];
 #pragma unroll
   for (int u = 0; u < A2_SV; ++u) sv[u] = sc[min(tid + NT * u, count - 1)];  // clamped, unconditional
-  float tv[3];  // wave 0, lane j < AC: column j's values past the fours (at most 3)
-  if (wave == 0) {
+  // waves 0-3, the 16 lanes of a row: a column's sum, and its values past the fours (at most 3)
+  const int col = (wave & 3) * 4 + (lane >> 4);
+  float tv[3];
+  if (wave < 4) {
 #pragma unroll
     for (int r = 0; r < 3; ++r)
-      tv[r] = cache1<HALF>(a.vcache, vcol + (int64_t)(lane % AC) * a.vstride + min(count4 + r, count - 1));
+      tv[r] = cache1<HALF>(a.vcache, vcol + (int64_t)col * a.vstride + min(count4 + r, count - 1));
   }
   if (wave == 0) {
     float mx = wmax(tmr[0], tmr[1]);
@@ -365,12 +378,13 @@ __global__ __launch_bounds__(A2_NT) void attend2_kernel(const AttnArgs a) {
         const int i = base + tid + NT * u;
         if (i < count) {
           const float d = sv[u] - mx;
-          if (i < count4) e4[(i & 3) * rs + (i >> 2)] = vexp(d);
+          if (i < count4) e4[(i & 3) * rs + chain16_at(i >> 2)] = vexp(d);
           else tail[i - count4] = fexp(d);
         }
       }
     }
   }
+  pad_rows(e4, 4, rs, q4, tid);
   __syncthreads();
   // the first pass's values requested now (clamped into the column: never used past q4): they fly while wave 0 runs
   // the exponentials' ordered sum (its reads 32 values at a time, so that both fit the registers)
@@ -381,25 +395,20 @@ __global__ __launch_bounds__(A2_NT) void attend2_kernel(const AttnArgs a) {
     for (int j = 0; j < AC; ++j) v0[j] = cache4<HALF>(a.vcache, vcol + (int64_t)j * a.vstride + 4 * bc);
   }
   if (wave == 0) {
-    // lanes 0-3: lane k's sum; ((l0 + l1) + l2) + l3, the tail in order, 1 / sum
-    const float part = lane < 4 ? lds_chain_h<4>(e4 + lane * rs, q4, 0.0f) : 0.0f;
-    const float c1 = __shfl(part, 1, 64), c2 = __shfl(part, 2, 64), c3 = __shfl(part, 3, 64);
-    if (lane == 0) {
-      float sum = ((part + c1) + c2) + c3;
-      for (int r = 0; r < count - count4; ++r) sum = sum + tail[r];
-      shared_inv = 1.0f / sum;
-    }
+    const float inv = inverse_sum(e4, rs, q4, tail, count - count4, lane);
+    if (lane == 0) shared_inv = inv;
   }
   __syncthreads();
   const float inv = shared_inv;
   // block b's products: (p0 v0 + p1 v1) + (p2 v2 + p3 v3) for the 16 columns, into the columns' rows
   auto products = [&](int b, const float4 (&v)[AC]) {
     if (b < q4) {
-      const float p0 = e4[b] * inv, p1 = e4[rs + b] * inv, p2 = e4[2 * rs + b] * inv, p3 = e4[3 * rs + b] * inv;
+      const int bs = chain16_at(b);
+      const float p0 = e4[bs] * inv, p1 = e4[rs + bs] * inv, p2 = e4[2 * rs + bs] * inv, p3 = e4[3 * rs + bs] * inv;
 #pragma unroll
       for (int j = 0; j < AC; ++j) {
         const float4 x = v[j];
-        blk[j * rs + b] = (p0 * x.x + p1 * x.y) + (p2 * x.z + p3 * x.w);
+        blk[j * rs + bs] = (p0 * x.x + p1 * x.y) + (p2 * x.z + p3 * x.w);
       }
     }
   };
@@ -411,13 +420,189 @@ __global__ __launch_bounds__(A2_NT) void attend2_kernel(const AttnArgs a) {
     for (int j = 0; j < AC; ++j) v[j] = cache4<HALF>(a.vcache, vcol + (int64_t)j * a.vstride + 4 * bc);
     products(b, v);
   }
+  pad_rows(blk, AC, rs, q4, tid);
   __syncthreads();
-  if (wave == 0 && lane < AC) {
-    float acc = lds_chain(blk + lane * rs, q4, 0.0f);
+  if (wave < 4) {
+    float acc = chain16_registers<true>(blk + col * rs, q4, lane & 15);
 #pragma unroll
     for (int r = 0; r < 3; ++r)
       if (r < count - count4) acc = acc + (tail[r] * inv) * tv[r];
-    a.out[(int64_t)t * a.out_stride + h * HS + j0 + lane] = acc;
+    if ((lane & 15) == (((q4 + 31) >> 5) & 15)) a.out[(int64_t)t * a.out_stride + h * HS + j0 + col] = acc;
+  }
+}
+
+template <int HS, bool HALF>
+__global__ __launch_bounds__(A2_NT) void attend2_kernel(const AttnArgs a) {
+  extern __shared__ float4 lds4[];
+  attend2<HS, HALF>(a, reinterpret_cast<float *>(lds4));
+}
+
+// (B + C) for a few tokens (decode) of long contexts whose output the caller quantizes itself: one block of 16 waves a
+// (token, query head, 16 columns), the exponentials in LDS as attend2_kernel, the weighted values in chunks of A3_BLOCKS
+// four-position blocks through two LDS buffers. Waves 4-15 make a chunk's four-position products (64 blocks and 4 columns
+// a wave, the values requested three chunks ahead) while waves 0-3 read the chunk before it into registers, a column a DPP
+// row of 16 lanes, and add the one before that (chain16). Bound by the two ordered sums of count / 4 steps, about 5 cycles
+// a step, and the values' way from the L2 (18 TB/s: every head of a kv head reads them). With the scores, from the caches:
+// 20,010 positions, 28 / 4 heads of 128, 50.4 us against 63.9 for attend_kernel, whose one wave adds 32 columns from LDS;
+// 8200 positions 26.9 against 33.9; 2060 positions, 32 / 8 heads, 12.8 against 15.6. A replayed decode step's launch is fixed by
+// the model's longest context: a block whose count fits attend2's LDS (up to `most2` positions) takes its steps.
+constexpr int A3_NT = 1024;      // threads a block
+constexpr int A3_BLOCKS = 192;   // four-position blocks a chunk: 6 segments of 32 a column (32,768 positions fit the LDS)
+constexpr int A3_SV = 16;        // scores a thread a pass
+constexpr int A3_AHEAD = 3;      // chunks of values a producer holds
+
+// LDS bytes of attend3_kernel for the largest count of a launch
+size_t attend3_lds(int count) {
+  return sizeof(float) * (size_t)(4 * chain_rowstride((count & ~3) >> 2) + 4 + 2 * A2_AC * A3_BLOCKS);
+}
+
+// four values of the cache as they lie there, and as float32
+template <bool HALF> struct Raw4 { typedef float4 T; };
+template <> struct Raw4<true> { typedef uint2 T; };
+__device__ __forceinline__ float4 float4_of(float4 v) { return v; }
+__device__ __forceinline__ float4 float4_of(uint2 h) {
+  return make_float4(from_f16((uint16_t)(h.x & 0xffff)), from_f16((uint16_t)(h.x >> 16)),
+                     from_f16((uint16_t)(h.y & 0xffff)), from_f16((uint16_t)(h.y >> 16)));
+}
+
+template <int HS, bool HALF>
+__global__ __launch_bounds__(A3_NT) void attend3_kernel(const AttnArgs a, const int most2) {
+  constexpr int NT = A3_NT, AC = A2_AC, S = HS / AC, CB = A3_BLOCKS, PC = 4;  // PC: columns a producer
+  constexpr int SEGS = CB / 32, D = A3_AHEAD;
+  static_assert((NT / 64 - 4) * 64 * PC == CB * AC, "the producers make a chunk");
+  typedef typename Raw4<HALF>::T Raw;
+  extern __shared__ float4 lds4[];
+  float *const lds = reinterpret_cast<float *>(lds4);
+  if (first_position(a) + (int)blockIdx.z + 1 <= most2) {  // uniform
+    attend2<HS, HALF>(a, lds);
+    return;
+  }
+  __shared__ float wave_mx[NT / 64], shared_inv;
+  const int mul = a.nh / a.nkv, groups = a.nkv * S;
+  const int xcd = blockIdx.x & 7, idx = blockIdx.x >> 3, hl = idx % mul, g = (idx / mul) * 8 + xcd;
+  if (g >= groups) return;  // the grid's rounding up: whole blocks leave
+  const int kh = g / S, j0 = (g % S) * AC, h = kh * mul + hl;
+  const int t = blockIdx.z, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int count = first_position(a) + t + 1, count4 = count & ~3, q4 = count4 >> 2, rs = chain_rowstride(q4);
+  float *const e4 = lds;             // [4][rs]
+  float *const tail = lds + 4 * rs;  // [4]
+  float *const buffers = tail + 4;   // [2][AC][CB]
+  const float *sc = a.scores + ((int64_t)t * a.nh + h) * a.seq_len;
+  const int64_t vcol = (int64_t)(kh * HS + j0) * a.vstride;  // the block's first value column
+  const int tiles = (count + TILE - 1) / TILE;
+  const float *tm = a.tilemax + ((int64_t)t * a.nh + h) * (a.seq_len / TILE + 1);
+  float mx = tm[min(tid, tiles - 1)];  // clamped: a repeat changes no max
+  float sv[A3_SV];
+#pragma unroll
+  for (int u = 0; u < A3_SV; ++u) sv[u] = sc[min(tid + NT * u, count - 1)];  // clamped, unconditional
+  const int col = (wave & 3) * 4 + (lane >> 4), l16 = lane & 15;  // waves 0-3: a column a row of 16 lanes
+  float tv[3];                                                    // and its values past the fours (at most 3)
+  if (wave < 4) {
+#pragma unroll
+    for (int r = 0; r < 3; ++r)
+      tv[r] = cache1<HALF>(a.vcache, vcol + (int64_t)col * a.vstride + min(count4 + r, count - 1));
+  }
+  for (int i = tid + NT; i < tiles; i += NT) mx = wmax(mx, tm[i]);
+  for (int o = 32; o >= 1; o >>= 1) mx = wmax(mx, __shfl_xor(mx, o, 64));
+  if (lane == 0) wave_mx[wave] = mx;
+  lds_barrier();
+  mx = wave_mx[0];
+#pragma unroll
+  for (int w = 1; w < NT / 64; ++w) mx = wmax(mx, wave_mx[w]);
+  // position tid + NT u of a pass lies NT / 4 floats after position tid + NT (u - 1)'s place (chain16_at keeps whole 256s)
+  static_assert(NT / 4 % 256 == 0, "chain16_at's turns repeat every 256 values");
+  float *const to0 = e4 + (tid & 3) * rs + chain16_at(tid >> 2);
+  for (int base = 0; base < count; base += NT * A3_SV) {
+    if (base > 0) {
+#pragma unroll
+      for (int u = 0; u < A3_SV; ++u) sv[u] = sc[min(base + tid + NT * u, count - 1)];
+    }
+#pragma unroll
+    for (int u = 0; u < A3_SV; ++u) {
+      const int i = base + tid + NT * u;
+      if (base + NT * (u + 1) <= count4) {  // (scalar branches: whole passes, then the one that the fours end in)
+        to0[(base + NT * u) / 4] = vexp(sv[u] - mx);
+      } else if (base + NT * u < count) {
+        if (i < count4) to0[(base + NT * u) / 4] = vexp(sv[u] - mx);
+        else if (i < count) tail[i - count4] = fexp(sv[u] - mx);
+      }
+    }
+  }
+  pad_rows(e4, 4, rs, q4, tid);
+  lds_barrier();
+  // a producer's four-position block of a chunk and its 4 columns (clamped into the columns: past q4 they become 0)
+  const bool producer = wave >= 4;  // uniform
+  const int pw = max(wave - 4, 0), pb = pw % (CB / 64) * 64 + lane, pj = pw / (CB / 64) * PC;
+  const Raw *const values = reinterpret_cast<const Raw *>(a.vcache) + (vcol + (int64_t)pj * a.vstride) / 4;
+  Raw held[D][PC];
+  auto fetch = [&](int c, Raw (&v)[PC]) {
+    const uint32_t at = max(min(c * CB + pb, q4 - 1), 0);  // (a scalar base a column, one offset a lane)
+#pragma unroll
+    for (int j = 0; j < PC; ++j) v[j] = (values + (int64_t)j * (a.vstride / 4))[at];
+  };
+  if (wave == 0) {
+    const float inv = inverse_sum(e4, rs, q4, tail, count - count4, lane);
+    if (lane == 0) shared_inv = inv;
+  } else if (producer) {  // (in flight meanwhile)
+#pragma unroll
+    for (int k = 0; k < D; ++k) fetch(k, held[k]);
+  }
+  lds_barrier();
+  const float inv = shared_inv;
+  const int chunks = (q4 + CB - 1) / CB;
+  // Step c of all waves, a barrier after each: chunk c's products into buffer c % 2 (its last readers passed the barrier
+  // before), chunk c - 1 from its buffer into registers, and chunk c - 2's adds
+  float *const to = buffers + pj * CB + chain16_at(pb);
+  auto produce = [&](int c, Raw (&v)[PC]) {
+    const int b = c * CB + pb, bs = chain16_at(min(b, q4 - 1));
+    const float p0 = e4[bs] * inv, p1 = e4[rs + bs] * inv, p2 = e4[2 * rs + bs] * inv, p3 = e4[3 * rs + bs] * inv;
+    float *const d = to + (c & 1) * (AC * CB);
+#pragma unroll
+    for (int j = 0; j < PC; ++j) {
+      const float4 x = float4_of(v[j]);
+      const float p = (p0 * x.x + p1 * x.y) + (p2 * x.z + p3 * x.w);
+      d[j * CB] = b < q4 ? p : 0.0f;
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    fetch(c + D, v);
+  };
+  float acc = 0.0f;
+  float4 ra[8], rb[8];
+  // (a chunk is 6 segments: chunk c's first starts on lane 6 c % 16 of the row)
+  auto take = [&](int c, float4 (&v)[8]) {
+    chain16_read(buffers + (c & 1) * (AC * CB) + col * CB, 0, SEGS, (l16 - SEGS * c) & 15, v);
+  };
+  auto add = [&](int c, float4 (&v)[8]) { acc = chain16_rounds<SEGS>(acc, v, (min(CB, q4 - c * CB) + 31) >> 5); };
+  // (a loop a role, the same barriers in each: the roles' registers are never live together)
+  const int steps = chunks ? 2 + ((chunks + 1) & ~1) : 0;
+  if (producer) {
+    for (int c = 0; c < steps; c += D) {
+#pragma unroll
+      for (int k = 0; k < D; ++k) {
+        if (c + k < chunks) produce(c + k, held[k]);
+        if (c + k < steps) lds_barrier();
+      }
+    }
+  } else {
+    if (chunks) {
+      lds_barrier();
+      take(0, ra);
+      lds_barrier();
+    }
+    for (int c = 1; c <= chunks; c += 2) {  // steps c + 1 and c + 2 (past the last chunk: the last read again, not added)
+      take(min(c, chunks - 1), rb);
+      add(c - 1, ra);
+      lds_barrier();
+      take(min(c + 1, chunks - 1), ra);
+      if (c < chunks) add(c, rb);
+      lds_barrier();
+    }
+  }
+  if (wave < 4) {
+#pragma unroll
+    for (int r = 0; r < 3; ++r)
+      if (r < count - count4) acc = acc + (tail[r] * inv) * tv[r];
+    if (l16 == (((q4 + 31) >> 5) & 15)) a.out[(int64_t)t * a.out_stride + h * HS + j0 + col] = acc;
   }
 }
 
@@ -463,11 +648,13 @@ __global__ __launch_bounds__(A2_NT) void attend1_kernel(const AttnArgs a) {
   const int b = tid & 255, cg = tid >> 8, bc = max(min(b, q4 - 1), 0);
 #pragma unroll
   for (int j = 0; j < 4; ++j) v[j] = cache4<HALF>(a.vcache, vcol + (int64_t)(4 * cg + j) * a.vstride + 4 * bc);
-  float tv[3];  // wave 0, lane j < AC: column j's values past the fours (at most 3)
-  if (wave == 0) {
+  // waves 0-3, the 16 lanes of a row: a column's sum, and its values past the fours (at most 3)
+  const int col = (wave & 3) * 4 + (lane >> 4);
+  float tv[3];
+  if (wave < 4) {
 #pragma unroll
     for (int r = 0; r < 3; ++r)
-      tv[r] = cache1<HALF>(a.vcache, vcol + (int64_t)(lane % AC) * a.vstride + min(count4 + r, count - 1));
+      tv[r] = cache1<HALF>(a.vcache, vcol + (int64_t)col * a.vstride + min(count4 + r, count - 1));
   }
   lds_barrier();  // (the queries; the loads stay in flight)
   float sc = -__builtin_inff();
@@ -498,34 +685,31 @@ __global__ __launch_bounds__(A2_NT) void attend1_kernel(const AttnArgs a) {
   for (int w = 1; w < 16; ++w) mx = wmax(mx, wave_mx[w]);
   if (tid < count) {
     const float d = sc - mx;
-    if (tid < count4) e4[(tid & 3) * rs + (tid >> 2)] = vexp(d);
+    if (tid < count4) e4[(tid & 3) * rs + chain16_at(tid >> 2)] = vexp(d);
     else tail[tid - count4] = fexp(d);
   }
+  pad_rows(e4, 4, rs, q4, tid);
   lds_barrier();
   if (wave == 0) {
-    // lanes 0-3: lane k's sum; ((l0 + l1) + l2) + l3, the tail in order, 1 / sum
-    const float part = lane < 4 ? lds_chain_h<4>(e4 + lane * rs, q4, 0.0f) : 0.0f;
-    const float c1 = __shfl(part, 1, 64), c2 = __shfl(part, 2, 64), c3 = __shfl(part, 3, 64);
-    if (lane == 0) {
-      float sum = ((part + c1) + c2) + c3;
-      for (int r = 0; r < count - count4; ++r) sum = sum + tail[r];
-      shared_inv = 1.0f / sum;
-    }
+    const float inv = inverse_sum(e4, rs, q4, tail, count - count4, lane);
+    if (lane == 0) shared_inv = inv;
   }
   lds_barrier();
   const float inv = shared_inv;
   if (b < q4) {
-    const float p0 = e4[b] * inv, p1 = e4[rs + b] * inv, p2 = e4[2 * rs + b] * inv, p3 = e4[3 * rs + b] * inv;
+    const int bs = chain16_at(b);
+    const float p0 = e4[bs] * inv, p1 = e4[rs + bs] * inv, p2 = e4[2 * rs + bs] * inv, p3 = e4[3 * rs + bs] * inv;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) blk[(4 * cg + j) * rs + b] = (p0 * v[j].x + p1 * v[j].y) + (p2 * v[j].z + p3 * v[j].w);
+    for (int j = 0; j < 4; ++j) blk[(4 * cg + j) * rs + bs] = (p0 * v[j].x + p1 * v[j].y) + (p2 * v[j].z + p3 * v[j].w);
   }
+  pad_rows(blk, AC, rs, q4, tid);
   lds_barrier();
-  if (wave == 0 && lane < AC) {
-    float acc = lds_chain(blk + lane * rs, q4, 0.0f);
+  if (wave < 4) {
+    float acc = chain16_registers<false>(blk + col * rs, q4, lane & 15);
 #pragma unroll
     for (int r = 0; r < 3; ++r)
       if (r < count - count4) acc = acc + (tail[r] * inv) * tv[r];
-    a.out[(int64_t)t * a.out_stride + h * HS + j0 + lane] = acc;
+    if ((lane & 15) == (((q4 + 31) >> 5) & 15)) a.out[(int64_t)t * a.out_stride + h * HS + j0 + col] = acc;
   }
 }
 
@@ -552,6 +736,17 @@ int attend_lds(const AttnArgs &a, int *nslot) {
 bool attend2_takes(const AttnArgs &a) {
   const int count = a.pos0 + a.m;
   return a.hs % A2_AC == 0 && count <= A2_MOST && attend2_lds(count) <= (size_t)ALDS;
+}
+
+// the largest count that attend2 takes in attend3_kernel's LDS for a launch of at most `count` positions
+int attend3_most2(int count) {
+  const int rs = (int)(attend3_lds(count) / sizeof(float) - 4) / (4 + A2_AC);  // floats a row
+  return std::min(A2_MOST, std::max(0, 4 * ((rs - 16) & ~63)));
+}
+
+// whether attend3_kernel takes a decode launch: head sizes of whole 16-column slices, a context that fits its LDS
+bool attend3_takes(const AttnArgs &a) {
+  return a.hs % A2_AC == 0 && attend3_lds(a.pos0 + a.m) <= (size_t)ALDS;
 }
 
 template <int HS, bool HALF>
@@ -583,6 +778,19 @@ hipError_t launch_hs(const AttnArgs &a, hipStream_t s) {
     }
     const int groups = a.nkv * (HS / A2_AC), g8 = (groups + 7) & ~7;
     hipLaunchKernelGGL((attend2_kernel<HS, HALF>), dim3(g8 * (a.nh / a.nkv), 1, a.m), dim3(A2_NT), lds, s, a);
+    return hipGetLastError();
+  }
+  if (a.m <= DECODE_TOKENS && !a.split && !a.xq && attend3_takes(a)) {
+    static bool sized = false;  // once a process: let the kernel take LDS past 64 KiB
+    if (!sized) {
+      const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&attend3_kernel<HS, HALF>),
+                                               hipFuncAttributeMaxDynamicSharedMemorySize, ALDS);
+      if (e != hipSuccess) return e;
+      sized = true;
+    }
+    const int groups = a.nkv * (HS / A2_AC), g8 = (groups + 7) & ~7;
+    hipLaunchKernelGGL((attend3_kernel<HS, HALF>), dim3(g8 * (a.nh / a.nkv), 1, a.m), dim3(A3_NT),
+                       attend3_lds(a.pos0 + a.m), s, a, attend3_most2(a.pos0 + a.m));
     return hipGetLastError();
   }
   int nslot = 0;

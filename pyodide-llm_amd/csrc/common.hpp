@@ -208,6 +208,72 @@ __device__ __forceinline__ float lds_chain_h(const float *c, int n, float acc) {
 }
 __device__ __forceinline__ float lds_chain(const float *c, int n, float acc) { return lds_chain_h<8>(c, n, acc); }
 
+// Where value i of an ordered sum lies in its LDS row for chain16_registers: 32 values a segment, a segment's float4 pieces
+// turned by the segment, so that the 16 lanes' reads of one step fall on distinct banks.
+__device__ __forceinline__ int chain16_at(int i) { return (i & ~31) | ((((i >> 2) ^ (i >> 5)) & 7) << 2) | (i & 3); }
+
+// An ordered sum run from registers by the 16 lanes of a DPP row (a wave runs four): 0 + c[0] + c[1] + ... in order, every
+// add rounded, over c = the sum's row of n values laid out by chain16_at (16-byte aligned), +0.0 from n up to the next
+// multiple of 32 (x + 0 is x for sums whose running values are never -0: they start at +0). Lane l holds segment l of 16,
+// 32 values; in every round each lane adds its values to what it has, and what it then has goes to the next lane (to the
+// first from the last), so that the lane whose turn it is starts from the true running sum, which is in lane
+// ceil(n / 32) % 16 of the row at the end. n is the same in the whole wave, and every lane of it is active. 5.1 cycles an
+// add (4.3 of them the dependent add), against 8.5 with the adds straight from LDS reads (lds_chain).
+// the 16 segments from `first` on, of `segs` in all (those past the last: read, never on the sum's way)
+__device__ __forceinline__ void chain16_read(const float *c, int first, int segs, int l16, float4 (&v)[8]) {
+  const int seg = min(first + l16, segs - 1);
+  const float4 *from = reinterpret_cast<const float4 *>(c + seg * 32);
+#pragma unroll
+  for (int u = 0; u < 8; ++u) v[u] = from[u ^ (seg & 7)];
+}
+// `last` rounds, at most 16 (unrolled by N: a loop's waits and branch cost half as much again as its 32 adds)
+template <int N = 8>
+__device__ __forceinline__ float chain16_rounds(float acc, float4 (&v)[8], int last) {
+#pragma unroll
+  for (int u = 0; u < 8; ++u) asm volatile("" : "+v"(v[u].x), "+v"(v[u].y), "+v"(v[u].z), "+v"(v[u].w));  // one wait
+  auto round = [&] {
+    acc = add32(acc, v);
+    acc = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(acc), 0x121, 0xF, 0xF, true));  // row_ror:1
+  };
+  last = min(last, 16);
+  int r = 0;
+  for (; r + N <= last; r += N) {
+#pragma unroll
+    for (int k = 0; k < N; ++k) round();
+  }
+  for (; r < last; ++r) round();
+  return acc;
+}
+// the whole sum; AHEAD: the next 16 segments are read while the present ones are added (32 registers more)
+template <bool AHEAD>
+__device__ __forceinline__ float chain16_registers(const float *c, int n, int l16) {
+  const int segs = (n + 31) >> 5;
+  float acc = 0.0f;
+  float4 v[8];
+  if (AHEAD) {
+    float4 w[8];
+    if (segs > 0) chain16_read(c, 0, segs, l16, v);
+    for (int first = 0; first < segs; first += 32) {
+      if (first + 16 < segs) chain16_read(c, first + 16, segs, l16, w);
+      acc = chain16_rounds(acc, v, segs - first);
+      if (first + 16 < segs) {
+        if (first + 32 < segs) chain16_read(c, first + 32, segs, l16, v);
+        acc = chain16_rounds(acc, w, segs - first - 16);
+      }
+    }
+  } else {
+    for (int first = 0; first < segs; first += 16) {
+      chain16_read(c, first, segs, l16, v);
+      acc = chain16_rounds(acc, v, segs - first);
+    }
+  }
+  return acc;
+}
+// chain16_registers' sum of row k of the wave (0..3), as a scalar
+__device__ __forceinline__ float chain16_result(float acc, int n, int k) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(acc), 16 * k + (((n + 31) >> 5) & 15)));
+}
+
 // An ordered sum run from registers by the 32 lanes of a half-wave: 0 + c[0] + c[1] + ... in order, every add
 // rounded, over c = the sum's row of values (16-byte aligned), +0.0 from its count up to 32 * nseg (x + 0 is x for sums
 // whose running values are never -0: they start at +0). Lane seg (0..31) of the half-wave is segment seg: in round
