@@ -946,7 +946,7 @@ namespace {
 // the graph of one decode step of a kind (the caller has run at least one step eagerly, so that every launch's one-time
 // set-up is done): captured with positions bounded by seq_len - 1 and read from state[STATE_POS]: the forward pass with
 // logits, the penalty over the window in device memory (STEP_PENALIZED), the greedy choice or the draw with the call's
-// settings and the round's random number (STEP_SAMPLED), then the step's end (launch_step_end)
+// settings and the round's random number (STEP_SAMPLED), whose last launch ends the step (StepEnd)
 void build_graph(he_engine *e, int kind) {
   e->graph_tried[kind] = true;
   // PYODIDE_LLM_HIP_GRAPH=0 keeps every step eager (a kernel-trace profiler that does not follow graph launches)
@@ -964,15 +964,13 @@ void build_graph(he_engine *e, int kind) {
       const bool drawn = (kind & STEP_SAMPLED) != 0, penalized = (kind & STEP_PENALIZED) != 0;
       // (a drawn step takes the penalty in the draw's first launch)
       if (penalized && !drawn) le = launch_penalize_steps(e->logits, e->window, e->state, e->run_params, e->stream);
+      const StepEnd end{e->logits, e->kept_logits, n, e->tokens, e->state, e->step_ids, e->step_values, e->window,
+                        e->run_params};
       if (le == hipSuccess)
         le = drawn ? launch_sample_steps(e->logits, n, e->run_params, e->state, penalized ? e->window : nullptr,
                                          (kind & STEP_WHOLE) != 0, e->sample_probs, e->sample_index,
-                                         e->sample_parts, e->sample_token, e->sample_best, e->stream)
-                   : launch_argmax(e->best_i, e->best_v, e->logits, n, e->amax_v, e->amax_i, e->stream);
-      if (le == hipSuccess)
-        le = launch_step_end(e->logits, n, e->kept_logits, e->tokens, e->state, drawn ? e->sample_token : e->best_i,
-                             drawn ? e->sample_best : e->best_v, e->step_ids, e->step_values, e->window,
-                             e->run_params, e->stream);
+                                         e->sample_parts, e->sample_token, e->sample_best, end, e->stream)
+                   : launch_argmax(e->best_i, e->best_v, e->logits, n, e->amax_v, e->amax_i, e->stream, end);
       if (le != hipSuccess) rc = HE_E_HIP;
     }
     const hipError_t end = hipStreamEndCapture(e->stream, &g);

@@ -207,9 +207,23 @@ hipError_t launch_valu_ceiling(int32_t passes, float w, float x0, float step, fl
 int32_t mfma_ceiling_waves();
 hipError_t launch_mfma_ceiling(int32_t passes, int32_t first, int32_t times, int32_t flip, uint32_t *out,
                                hipStream_t s);
+struct RunParams;
+// the end of a replayed step, by the launch that chooses its token (stepend.hpp): where this step ends the call (a stop
+// token, no token, a largest logit that is not finite) and none before it did, its logits into kept and
+// state[STATE_HALTED] = step + 1; its token and value into ids / values at the step, the token into the window and as the
+// next step's input (tokens[0]), the position and the step advanced. params null: no step to end.
+struct StepEnd {
+  const float *logits;
+  float *kept;
+  int32_t n;
+  int32_t *tokens, *state, *ids;
+  float *values;
+  int32_t *window;
+  const RunParams *params;
+};
 // greedy: the first index of the largest logit into *out (and the value into *value)
 hipError_t launch_argmax(int32_t *out, float *value, const float *x, int32_t n, float *scratch_v, int32_t *scratch_i,
-                         hipStream_t s);
+                         hipStream_t s, const StepEnd &end = StepEnd{});
 // the repetition penalty (kernels/kernel.ts:705-719) on the distinct tokens of tokens[0..count), count <= 64
 hipError_t launch_penalize(float *logits, const int32_t *tokens, int32_t count, float penalty, hipStream_t s);
 // one token drawn from softmax(logits / temperature) (kernels/kernel.ts:803-868) for random in [0, 1), restricted to
@@ -274,21 +288,13 @@ struct RunParams {
 // a step's draw (as launch_sample) with the call's temperature and top-p and the round's random number of the step;
 // with window, the call's penalty over the window's state[STATE_WINDOW] tokens first (launch_penalize_steps's, in the
 // draw's first launch: the logits penalized in place); whole: the call's top-p is known to take no nucleus (one launch
-// fewer)
+// fewer); end: the step's end, in the draw's last launch
 hipError_t launch_sample_steps(float *logits, int32_t n, const RunParams *params, const int32_t *state,
                                const int32_t *window, bool whole, float *probs, int32_t *index, DrawParts *parts,
-                               int32_t *out_token, float *out_best, hipStream_t s);
+                               int32_t *out_token, float *out_best, const StepEnd &end, hipStream_t s);
 // the call's penalty over the window's state[STATE_WINDOW] tokens
 hipError_t launch_penalize_steps(float *logits, const int32_t *window, const int32_t *state, const RunParams *params,
                                  hipStream_t s);
-// the end of a replayed step that chose *token (largest logit *value): where this step ends the call (a stop token,
-// no token, a largest logit that is not finite) and none before it did, its logits into kept and state[STATE_HALTED]
-// = step + 1; its token and value into ids / values at the step, the token into the window and as the next step's
-// input (tokens[0]), the position and the step advanced
-hipError_t launch_step_end(const float *logits, int32_t n, float *kept, int32_t *tokens, int32_t *state,
-                           const int32_t *token, const float *value, int32_t *ids, float *values, int32_t *window,
-                           const RunParams *params, hipStream_t s);
-
 // ---- the other forms (forms.hip) ----
 // layernorm (eps 1e-5) then quantize_x, m tokens; out (optional) the float32 rows; copy (optional, x_stride) x itself
 hipError_t launch_layernorm_quant(int8_t *xq, float *xs, float *out, float *copy, const float *x, const float *w,

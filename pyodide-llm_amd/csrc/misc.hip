@@ -10,6 +10,7 @@
 #include "common.hpp"
 #include "kernels.hpp"
 #include "l2fetch.hpp"
+#include "stepend.hpp"
 
 namespace ple {
 
@@ -329,8 +330,9 @@ __device__ __forceinline__ bool better(float v, int i, float bv, int bi) {
   if (bv != bv) return false;
   return v > bv || (v == bv && i < bi);
 }
+// (the last stage, one block, ends a replayed step too: end.params)
 __global__ __launch_bounds__(256) void argmax_stage(float *ov, int32_t *oi, const float *x, const int32_t *xi,
-                                                    int32_t n) {
+                                                    int32_t n, const StepEnd end) {
   __shared__ float sv[256];
   __shared__ int si[256];
   float bv = -__builtin_inff();
@@ -361,6 +363,7 @@ __global__ __launch_bounds__(256) void argmax_stage(float *ov, int32_t *oi, cons
     ov[blockIdx.x] = sv[0];
     oi[blockIdx.x] = si[0];
   }
+  if (end.params) step_end(end, si[0], sv[0], threadIdx.x, 256);
 }
 
 // ---- the device twin of the oracle's synthetic checkpoint (oracle/oracle.c or_synth_value, or_quantize,
@@ -501,12 +504,12 @@ hipError_t launch_qkv_post(const QkvPost &a, hipStream_t s) {
 }
 
 hipError_t launch_argmax(int32_t *out, float *value, const float *x, int32_t n, float *scratch_v, int32_t *scratch_i,
-                         hipStream_t s) {
+                         hipStream_t s, const StepEnd &end) {
   const int blocks = 256;
   hipLaunchKernelGGL(argmax_stage, dim3(blocks), dim3(256), 0, s, scratch_v, scratch_i, x, (const int32_t *)nullptr,
-                     n);
+                     n, StepEnd{});
   hipLaunchKernelGGL(argmax_stage, dim3(1), dim3(256), 0, s, value, out, (const float *)scratch_v,
-                     (const int32_t *)scratch_i, blocks);
+                     (const int32_t *)scratch_i, blocks, end);
   return hipGetLastError();
 }
 

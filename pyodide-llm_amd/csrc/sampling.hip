@@ -18,6 +18,7 @@
 
 #include "common.hpp"
 #include "kernels.hpp"
+#include "stepend.hpp"
 
 namespace ple {
 
@@ -1025,8 +1026,17 @@ __global__ __launch_bounds__(64) void chunk_sums_kernel(const float *p, DrawPart
 
 __global__ __launch_bounds__(ST) void draw_kernel(int32_t n, const DrawParts *parts, float *probs, int32_t *index,
                                                   int32_t *out_token, float *out_best, float temperature, float topp,
-                                                  double random, const RunParams *params, const int32_t *state) {
-  draw_block(n, settings(temperature, topp, random, params, state), parts, probs, index, out_token, out_best);
+                                                  double random, const RunParams *params, const int32_t *state,
+                                                  const StepEnd end) {
+  __shared__ int32_t token;
+  __shared__ float best;
+  draw_block(n, settings(temperature, topp, random, params, state), parts, probs, index, &token, &best);
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    *out_token = token;
+    *out_best = best;
+  }
+  if (end.params) step_end(end, token, best, threadIdx.x, ST);
 }
 
 // the five launches of a draw (the settings as values, or with params the call's and the step's from device memory;
@@ -1034,7 +1044,7 @@ __global__ __launch_bounds__(ST) void draw_kernel(int32_t n, const DrawParts *pa
 hipError_t launch_draw(const float *logits, int32_t n, float temperature, float topp, double random,
                        const RunParams *params, const int32_t *state, float *probs, int32_t *index, DrawParts *parts,
                        int32_t *out_token, float *out_best, hipStream_t s, float *write_back = nullptr,
-                       const int32_t *window = nullptr, bool whole = false) {
+                       const int32_t *window = nullptr, bool whole = false, const StepEnd &end = StepEnd{}) {
   const int blocks = (n + CHUNK - 1) / CHUNK;
   hipLaunchKernelGGL(vocab_max_kernel, dim3(blocks), dim3(VB), 0, s, logits, n, parts, write_back, window, state,
                      params, (int32_t)whole);
@@ -1046,7 +1056,7 @@ hipError_t launch_draw(const float *logits, int32_t n, float temperature, float 
   hipLaunchKernelGGL(vocab_guess_kernel, dim3(blocks), dim3(64 * GW), 0, s, n, parts, probs, temperature, topp, random,
                      params, state);
   hipLaunchKernelGGL(draw_kernel, dim3(1), dim3(ST), 0, s, n, parts, probs, index, out_token, out_best, temperature,
-                     topp, random, params, state);
+                     topp, random, params, state, end);
   return hipGetLastError();
 }
 
@@ -1062,75 +1072,19 @@ __global__ __launch_bounds__(64) void penalize_steps_kernel(float *logits, const
   logits[t] = v > 0 ? v / penalty : v * penalty;
 }
 
-// whether the step that chose `token` with largest logit `value` ends the call: a token that is not one (the draw's
-// SAMPLE_NOT_FINITE or SAMPLE_DECLINED), a largest logit that is not finite, or a stop token
-__device__ __forceinline__ bool halts(int32_t token, float value, const RunParams *params) {
-  if (token < 0 || !__builtin_isfinite(value)) return true;
-  const int ns = params->n_stops;
-  for (int j = 0; j < RUN_STOPS_MOST; ++j)
-    if (j < ns && params->stops[j] == token) return true;
-  return false;
-}
-
-// the logits of the step that ends the call, kept (the replays after it in the round overwrite the step's own)
-__global__ __launch_bounds__(256) void keep_halting_kernel(const float *logits, int32_t n, float *kept,
-                                                           const int32_t *token, const float *value,
-                                                           const int32_t *state, const RunParams *params) {
-  if (state[STATE_HALTED] != 0 || !halts(*token, *value, params)) return;  // (the same for every block)
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-    kept[i] = logits[i];
-}
-
-// the end of a replayed step: its token and largest logit into ids / values at the step, the halting step noted
-// (state[STATE_HALTED] = step + 1, the first one only), the token appended to the penalty's window (a ring of
-// REPETITION_WINDOW once full), the token made the next step's input (a valid one after a step that chose none), the
-// position and the step advanced
-__global__ void advance_steps_kernel(int32_t *tokens, int32_t *state, const int32_t *token, const float *value,
-                                     int32_t *ids, float *values, int32_t *window, const RunParams *params) {
-  const int32_t step = state[STATE_STEP], b = *token;
-  const float v = *value;
-  ids[step] = b;
-  values[step] = v;
-  if (state[STATE_HALTED] == 0 && halts(b, v, params)) state[STATE_HALTED] = step + 1;
-  if (b >= 0) {
-    const int32_t count = state[STATE_WINDOW];
-    if (count < RUN_WINDOW) {
-      window[count] = b;
-      state[STATE_WINDOW] = count + 1;
-    } else {
-      const int32_t head = state[STATE_HEAD];
-      window[head] = b;
-      state[STATE_HEAD] = head + 1 == RUN_WINDOW ? 0 : head + 1;
-    }
-  }
-  tokens[0] = b >= 0 ? b : 0;
-  state[STATE_POS] = state[STATE_POS] + 1;
-  state[STATE_STEP] = step + 1;
-}
-
 }  // namespace
 
 hipError_t launch_sample_steps(float *logits, int32_t n, const RunParams *params, const int32_t *state,
                                const int32_t *window, bool whole, float *probs, int32_t *index, DrawParts *parts,
-                               int32_t *out_token, float *out_best, hipStream_t s) {
+                               int32_t *out_token, float *out_best, const StepEnd &end, hipStream_t s) {
   if (n < 1 || n > SAMPLE_MOST) return hipErrorInvalidValue;
   return launch_draw(logits, n, 0.0f, 0.0f, 0.0, params, state, probs, index, parts, out_token, out_best, s,
-                     window ? logits : nullptr, window, whole);
+                     window ? logits : nullptr, window, whole, end);
 }
 
 hipError_t launch_penalize_steps(float *logits, const int32_t *window, const int32_t *state, const RunParams *params,
                                  hipStream_t s) {
   hipLaunchKernelGGL(penalize_steps_kernel, dim3(1), dim3(RUN_WINDOW), 0, s, logits, window, state, params);
-  return hipGetLastError();
-}
-
-hipError_t launch_step_end(const float *logits, int32_t n, float *kept, int32_t *tokens, int32_t *state,
-                           const int32_t *token, const float *value, int32_t *ids, float *values, int32_t *window,
-                           const RunParams *params, hipStream_t s) {
-  const int blocks = (int)std::min<int64_t>(128, ((int64_t)n + 1023) / 1024);
-  hipLaunchKernelGGL(keep_halting_kernel, dim3(blocks), dim3(256), 0, s, logits, n, kept, token, value, state, params);
-  hipLaunchKernelGGL(advance_steps_kernel, dim3(1), dim3(1), 0, s, tokens, state, token, value, ids, values, window,
-                     params);
   return hipGetLastError();
 }
 
