@@ -206,20 +206,40 @@ __device__ __forceinline__ int chunk_lanes(const float (&v)[SEG], double run, in
   return chunk_lanes_r(lane_r(v, binade(run)), run, from, start, end);
 }
 
+// the lane's 32 values added to acc in order, widened eight at a time (all 32 held widened would not fit beside the
+// callers' state; one at a time each add waits for its own conversion)
+__device__ __forceinline__ double add_values(const float (&v)[SEG], double acc) {
+#pragma unroll
+  for (int k = 0; k < SEG; k += 8) {
+    float t[8];
+    double d[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      t[u] = v[k + u];
+      asm volatile("" : "+v"(t[u]));
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u) d[u] = (double)t[u];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) acc = acc + d[u];
+  }
+  return acc;
+}
+
 // One chunk (values b.., lane L's 32 at b + 32 L) exactly from run, by one wave: the lanes in parallel while the sum
-// stays in one binade; a lane that takes it out of its binade, and the first lane while the sum is 0, adds its values
-// one after another; then the lanes after it in parallel again. After two such lanes (a sum that still crosses
-// binades often: a parallel pass costs about as much as twenty lanes' adds in turn) the rest of the chunk goes lane
-// by lane, each adding its values to the sum the lane below hands it. Returns the chunk's end (every lane); with cp,
-// the checkpoints of the chunk's values.
+// stays in one binade; a lane that takes it out of its binade adds its values one after another; then the lanes after
+// it in parallel again. After two such lanes (a sum that still crosses binades often: a parallel pass costs about as
+// much as twenty lanes' adds in turn), and from a sum of 0, the rest of the chunk goes lane by lane. Returns the
+// chunk's end (every lane); with cp, the checkpoints of the chunk's values. (A nucleus draw's total of 1091 kept values,
+// one chunk from 0: 48,000 -> 13,400 cycles with the turns past the last value left out, no parallel pass from 0, and the
+// conversions out of the chain.)
 __device__ __forceinline__ double chunk_exact(const float (&v)[SEG], double run, int b, int count, double *cp) {
   const int lane = threadIdx.x & 63;
   double pre = 0.0;  // this lane's sum before its values
   int from = 0;
-  for (int crossed = 0; from < 64 && crossed < 2; ++crossed) {
-    int cross = from;
+  for (int crossed = 0; run > 0.0 && from < 64 && crossed < 2; ++crossed) {
     double start = run, end = 0.0;
-    if (run > 0.0) cross = chunk_lanes(v, run, from, &start, &end);
+    const int cross = chunk_lanes(v, run, from, &start, &end);
     if (lane >= from && lane <= cross) pre = start;
     if (cross == 64) {
       run = uniform(end);
@@ -227,28 +247,25 @@ __device__ __forceinline__ double chunk_exact(const float (&v)[SEG], double run,
       break;
     }
     // lane cross's values in order from its start (every lane adds its own; lane cross's sum is kept)
-    double acc = from_lane(start, cross);
-#pragma unroll
-    for (int u = 0; u < SEG; ++u) {
-      float t = v[u];
-      asm volatile("" : "+v"(t));  // (widened here, one at a time: all 32 held widened would not fit)
-      acc = acc + (double)t;
-    }
+    const double acc = add_values(v, from_lane(start, cross));
     run = from_lane(acc, cross);
     from = cross + 1;
   }
-  // lane by lane: in turn s lane s adds its values to the sum in acc (every lane adds its own; lane s + 1 takes lane
-  // s's sum, by a readlane: the turns are few enough here that the hand-on's latency does not matter)
-  for (int s = from; s < 64; ++s) {
-    if (lane == s) pre = run;
-    double acc = run;
+  // lane by lane: in turn s lane s adds its values to the sum the lane below handed it (every lane adds its own, all
+  // widened before the first turn), up to the last lane with a value of the chunk (+0.0 past it changes no sum)
+  const int lanes = min(64, (count - b + SEG - 1) / SEG);
+  if (from < lanes) {
+    double d[SEG], acc = run;
 #pragma unroll
-    for (int u = 0; u < SEG; ++u) {
-      float t = v[u];
-      asm volatile("" : "+v"(t));
-      acc = acc + (double)t;
+    for (int u = 0; u < SEG; ++u) d[u] = (double)v[u];
+    for (int s = from;; ++s) {
+      if (lane == s) pre = acc;
+#pragma unroll
+      for (int u = 0; u < SEG; ++u) acc = acc + d[u];
+      if (s + 1 >= lanes) break;
+      acc = lane_below(acc);
     }
-    run = from_lane(acc, s);
+    run = from_lane(acc, lanes - 1);
   }
   if (cp && lane % (CP_BLOCK / SEG) == 0 && b + SEG * lane < count) cp[(b + SEG * lane) / CP_BLOCK] = pre;
   return run;
@@ -258,14 +275,7 @@ __device__ __forceinline__ double chunk_exact(const float (&v)[SEG], double run,
 // lane from's pre (its sum before them) set to run
 __device__ __forceinline__ double lane_in_order(const float (&v)[SEG], double run, int from, double &pre) {
   if ((int)(threadIdx.x & 63) == from) pre = run;
-  double acc = run;
-#pragma unroll
-  for (int u = 0; u < SEG; ++u) {
-    float t = v[u];
-    asm volatile("" : "+v"(t));
-    acc = acc + (double)t;
-  }
-  return from_lane(acc, from);
+  return from_lane(add_values(v, run), from);
 }
 
 // One chunk (values b.., lane L's 32 at b + 32 L) exactly from run > 0 at lane from (the lanes below it done, their
@@ -294,13 +304,7 @@ __device__ __forceinline__ bool chunk_walk(const float (&v)[SEG], double run, in
       break;
     }
     // lane cross's values in order from its start (every lane adds its own; lane cross's sum is kept)
-    double acc = from_lane(start, cross);
-#pragma unroll
-    for (int u = 0; u < SEG; ++u) {
-      float t = v[u];
-      asm volatile("" : "+v"(t));
-      acc = acc + (double)t;
-    }
+    const double acc = add_values(v, from_lane(start, cross));
     run = from_lane(acc, cross);
     from = cross + 1;
   }
@@ -963,24 +967,41 @@ __device__ __forceinline__ void draw_block(int32_t n, const Settings &st, const 
     si[j] = 0x7fffffff;
   }
   __syncthreads();
-  // bitonic sort of size pairs into the order of before()
-  for (int width = 2; width <= size; width <<= 1) {
-    for (int stride = width >> 1; stride > 0; stride >>= 1) {
-      for (int j = tid; j < size; j += ST) {
-        const int partner = j ^ stride;
-        if (partner > j) {
-          const bool forward = (j & width) == 0;
-          const float pa = sp[j], pb = sp[partner];
-          const int ia = si[j], ib = si[partner];
-          if (before(pb, ib, pa, ia) == forward) {
-            sp[j] = pb;
-            si[j] = ib;
-            sp[partner] = pa;
-            si[partner] = ia;
+  // sorted into the order of before(): up to 64 pairs by wave 0, each lane counting the pairs before its own (19 pairs:
+  // 7200 -> 2600 cycles; a step of the block's bitonic sort is a block barrier), more by a bitonic sort of size pairs
+  if (likely <= 64) {
+    if (wave == 0) {
+      const float p = sp[min(lane, likely - 1)];
+      const int id = si[min(lane, likely - 1)];
+      int rank = 0;
+      for (int j = 0; j < likely; ++j)
+        rank += before(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(p), j)), __builtin_amdgcn_readlane(id, j), p, id);
+      wave_sync_lds();
+      if (lane < likely) {
+        sp[rank] = p;
+        si[rank] = id;
+      }
+      wave_sync_lds();
+    }
+  } else {
+    for (int width = 2; width <= size; width <<= 1) {
+      for (int stride = width >> 1; stride > 0; stride >>= 1) {
+        for (int j = tid; j < size; j += ST) {
+          const int partner = j ^ stride;
+          if (partner > j) {
+            const bool forward = (j & width) == 0;
+            const float pa = sp[j], pb = sp[partner];
+            const int ia = si[j], ib = si[partner];
+            if (before(pb, ib, pa, ia) == forward) {
+              sp[j] = pb;
+              si[j] = ib;
+              sp[partner] = pa;
+              si[partner] = ia;
+            }
           }
         }
+        __syncthreads();
       }
-      __syncthreads();
     }
   }
   if (tid == 0) {
