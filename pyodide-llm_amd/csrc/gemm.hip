@@ -320,7 +320,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2))) void ge
     glu_epilogue(a, out, reinterpret_cast<float *>(&stage[0]), r0, t0, wave, lane);
     return;
   }
-  // y[t][r] = out (or y + out): the lane's two tokens, its 16 rows in 4 runs of 4
+  // y[t][r] = out (or y + out), + bias: the lane's two tokens, its 16 rows in 4 runs of 4
+  const bool biased = a.seg[0].bias || a.seg[1].bias || a.seg[2].bias;  // (uniform: most launches have none)
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
     const int t = t0 + wt * 64 + h * 32 + (lane & 31);
@@ -341,10 +342,13 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2))) void ge
       float *y = (si == 2 ? a.seg[2].y : si == 1 ? a.seg[1].y : a.seg[0].y);
       const int stride = (si == 2 ? a.seg[2].y_stride : si == 1 ? a.seg[1].y_stride : a.seg[0].y_stride);
       const int accumulate = (si == 2 ? a.seg[2].accumulate : si == 1 ? a.seg[1].accumulate : a.seg[0].accumulate);
-      const float *bias = (si == 2 ? a.seg[2].bias : si == 1 ? a.seg[1].bias : a.seg[0].bias);
       float *dst = y + (int64_t)t * stride + r;
-      const float o = accumulate ? *dst + out[h][v] : out[h][v];
-      *dst = bias ? o + bias[r] : o;
+      float o = accumulate ? *dst + out[h][v] : out[h][v];
+      if (biased) {
+        const float *bias = (si == 2 ? a.seg[2].bias : si == 1 ? a.seg[1].bias : a.seg[0].bias);
+        if (bias) o = o + bias[r];
+      }
+      *dst = o;
     }
   }
 }
