@@ -941,7 +941,8 @@ __device__ __forceinline__ void draw_block(int32_t n, const Settings &st, const 
   int at = block_scan(lane == 0 ? lc : 0, wi, &shared_likely);
   at = __shfl(at, 0, 64);
   const int likely = shared_likely;
-  if (likely > SORT_MOST) {
+  // (none where 1 / temperature is past float32: largest logits that tie are then NaN, and no p is left to sort)
+  if (likely < 1 || likely > SORT_MOST) {
     if (tid == 0) {
       *out_token = SAMPLE_DECLINED;
       *out_best = best;

@@ -18,3 +18,10 @@ def test_small_nucleus_draws(n, spread):
     for topp in (0.05, 0.5, 0.95):
         for random in (0.0, 0.3, 0.77, 0.999999):
             assert gl.sample(logits, 0.8, topp, random) == ol.sample(logits, 0.8, topp, random), (topp, random)
+
+
+@pytest.mark.parametrize("n", [4, 8, 64, 2052])
+def test_nothing_kept(n):
+    """equal logits at a temperature whose reciprocal is past float32: 0 * infinity, no probability to sort. Declined: the
+    caller takes the step (the reference's own loop reads before its list here, so there is no token to compare)"""
+    assert gl.sample(np.full(n, 3.0, np.float32), 1e-40, 0.5, 0.3) == -2
