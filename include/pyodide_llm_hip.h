@@ -176,7 +176,7 @@ int32_t he_close(he_engine *e);
 
 /* The kinds of kernel he_profile_forward reports on */
 enum {
-  HE_K_GEMV = 0,   /* the decode matmuls (one token; bias 0: a few) */
+  HE_K_GEMV = 0,   /* the decode matmuls (one token, or a few) */
   HE_K_GEMM,       /* the matmuls of more tokens, on MFMA */
   HE_K_ATTENTION,  /* scores, softmax, weighted values */
   HE_K_NORM,       /* rmsnorm with quantize_x, quantize_x alone */
@@ -216,7 +216,8 @@ int32_t hk_quantize_x(void *xq, void *xs, const void *x, int32_t m, int32_t n, i
  * group scales ws [rows][K/32], against activations xq [m][K] / xs [m][K/32] from hk_quantize_x with the same bias:
  * matmul_q8r (kernels/kernel_relaxed.ts:34-67) for bias 64, matmul_q8 (kernels/kernel.ts:231-258) for bias 0,
  * matmul_q6r / matmul_q6 for int6; matmul_q8r_tile (kernels/kernel_relaxed.ts:164-183) is the same per token.
- * y is [m][rows] float32. One token (bias 0: a few) runs the decode GEMV, more the MFMA GEMM; both give the same bits. */
+ * y is [m][rows] float32. One token, or a few against few or long rows, runs the decode GEMV, the rest the MFMA GEMM: the
+ * same bits. */
 int32_t hk_matmul(void *y, const void *xq, const void *xs, const void *w, const void *ws, int32_t m, int32_t rows,
                   int32_t k, int32_t bias, int32_t six, void *stream);
 

@@ -28,11 +28,12 @@ namespace {
 
 thread_local std::string g_error;
 
-// whether m tokens against rows of k go to the GEMM: more than the GEMV takes (rows that it does not take at all: more
-// than 8 tokens of bias 64, the rest is refused)
-bool on_gemm(int32_t k, int32_t m, bool relaxed) {
-  const int32_t most = gemv_tokens(k, relaxed);
-  return most < 1 ? relaxed && m > 8 : m > most;
+// whether a matmul of m tokens against `rows` rows of k goes to the GEMM: where it is the faster of the two. (Rows that the
+// GEMV does not take, past 127 KiB with bias 64 and 31 KiB with bias 0: the interface takes more than 8 tokens of bias 64
+// and refuses the rest.)
+bool on_gemm(int32_t rows, int32_t k, int32_t m, bool six, bool relaxed) {
+  if (gemv_tokens(k, relaxed) < 1) return relaxed && m > 8;
+  return !gemv_faster(rows, k, m, six, relaxed);
 }
 
 int32_t fail(int32_t code, const std::string &what) {
@@ -516,8 +517,13 @@ hipError_t matmul_launch(he_engine *e, const MatSeg *segs, int nseg, int32_t k, 
   return launch_gemv(a, e->c.six, e->c.relaxed, e->stream);
 }
 
-// more tokens than one GEMV launch takes go to the MFMA GEMM (the same bits per token and row)
-bool use_gemm(const he_engine *e, int32_t k, int32_t m) { return on_gemm(k, m, e->c.relaxed != 0); }
+// whether a pass of m tokens takes the MFMA GEMM for the matmuls whose epilogues save launches (q / k / v, the FFN's
+// activation), against rows of k: from two tokens with bias 64, from seven with bias 0 (fewer where the GEMV takes fewer)
+bool use_gemm(const he_engine *e, int32_t k, int32_t m) {
+  const int32_t most = gemv_tokens(k, e->c.relaxed != 0);
+  if (most < 1) return e->c.relaxed && m > 8;
+  return m > (e->c.relaxed ? 1 : std::min(most, 6));
+}
 
 hipError_t gemm_launch(he_engine *e, const MatSeg *segs, int nseg, int32_t k, int32_t m, const int8_t *xq,
                        const float *xs, const QkvFuse *qkv) {
@@ -569,7 +575,10 @@ bool ffn_in_gemm(const he_engine *e, int32_t m) {
 
 hipError_t matmul(he_engine *e, const MatSeg *segs, int nseg, int32_t k, int32_t m, const int8_t *xq, const float *xs,
                   const F32Source *f32 = nullptr, const QkvFuse *qkv = nullptr, bool persistent = false) {
-  if (use_gemm(e, k, m))
+  int32_t rows = 0;
+  for (int i = 0; i < nseg; ++i) rows += segs[i].rows;
+  // (the GEMV finishes q / k / v of one token only)
+  if (qkv && m > 1 ? use_gemm(e, k, m) : on_gemm(rows, k, m, e->c.six != 0, e->c.relaxed != 0))
     return timed(e, HE_K_GEMM, matmul_bytes(e, segs, nseg, k, m),
                  [&] { return gemm_launch(e, segs, nseg, k, m, xq, xs, qkv); });
   return timed(e, HE_K_GEMV, matmul_bytes(e, segs, nseg, k, m),
@@ -1367,7 +1376,7 @@ int32_t hk_matmul(void *y, const void *xq, const void *xs, const void *w, const 
   if (!y || !xs || !ws) return fail(HE_E_ARG, "matmul: a required pointer is null");
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   base.m = m;
-  const bool gemm = on_gemm(k, m, bias == 64);
+  const bool gemm = on_gemm(rows, k, m, six != 0, bias == 64);
   if (!gemm && gemv_tokens(k, bias == 64) < 1) return fail(HE_E_ARG, "matmul: rows too long for the GEMV");
   HIP_TRY(gemm ? launch_gemm(base, six != 0, bias == 64, s) : launch_gemv(base, six != 0, bias == 64, s));
   return HE_OK;

@@ -1,5 +1,5 @@
-// gemv.hip — the decode matmul (one token; up to 6 with bias 0) of int8/int6 rows against quantized activations, to the bit of the
-// reference's CPU kernels:
+// gemv.hip — the decode matmul (one token, or a few: gemv_faster) of int8/int6 rows against quantized activations, to the bit of
+// the reference's CPU kernels:
 //   bias 64: kernels/kernel_relaxed.ts:34-67 matmul_q8r (and :195-218 matmul_q6r): per group the exact integer
 //            S_g = dot(w, q - 64); lane g % 4 of four float32 accumulators adds f32(S_g) * f32(ws * xs) for the groups
 //            in fours, in order; the lanes are added ((l0 + l1) + l2) + l3; the groups past the fours one at a time.
@@ -971,32 +971,64 @@ hipError_t launch_m(const MatArgs &a, hipStream_t s) {
 
 template <bool SIX, bool RELAXED, bool SUMS>
 hipError_t launch_sel(const MatArgs &a, hipStream_t s) {
-  if (a.m == 1) return launch_m<1, SIX, RELAXED, SUMS>(a, s);
-  if constexpr (SUMS || !RELAXED) {
-    switch (a.m) {
-      case 2: return launch_m<2, SIX, RELAXED, SUMS>(a, s);
-      case 3: return launch_m<3, SIX, RELAXED, SUMS>(a, s);
-      case 4: return launch_m<4, SIX, RELAXED, SUMS>(a, s);
-      case 5: return launch_m<5, SIX, RELAXED, SUMS>(a, s);
-      case 6: return launch_m<6, SIX, RELAXED, SUMS>(a, s);
-    }
+  switch (a.m) {
+    case 1: return launch_m<1, SIX, RELAXED, SUMS>(a, s);
+    case 2: return launch_m<2, SIX, RELAXED, SUMS>(a, s);
+    case 3: return launch_m<3, SIX, RELAXED, SUMS>(a, s);
+    case 4: return launch_m<4, SIX, RELAXED, SUMS>(a, s);
+    case 5: return launch_m<5, SIX, RELAXED, SUMS>(a, s);
+    case 6: return launch_m<6, SIX, RELAXED, SUMS>(a, s);
+    case 7: return launch_m<7, SIX, RELAXED, SUMS>(a, s);
+    case 8: return launch_m<8, SIX, RELAXED, SUMS>(a, s);
+    default: return hipErrorInvalidValue;
   }
-  if constexpr (SUMS) {
-    if (a.m == 7) return launch_m<7, SIX, RELAXED, SUMS>(a, s);
-    if (a.m == 8) return launch_m<8, SIX, RELAXED, SUMS>(a, s);
-  }
-  return hipErrorInvalidValue;
 }
 
 }  // namespace
 
 int32_t gemv_tokens(int32_t k, bool relaxed) {
-  // none where a block's products of one token pass 64 KiB of LDS. Bias 64: one token (two go to the GEMM: 4096 x 4096
-  // 8.2 against 10.7 us here, 4096 x 14336 21.1 against 22.1). Bias 0: up to 6, fewer where their products pass the LDS
-  // (4096 x 4096, 6 tokens 15.6 against 17.0 us in the GEMM, 8 tokens 24.4 against 17.0).
+  // 8, fewer where a block's products would pass 64 KiB of LDS
   const size_t per_token = sizeof(float) * WAVES * (size_t)row_layout(k, relaxed).stride;
-  const int32_t m = (int32_t)((64 * 1024) / per_token), most = relaxed ? 1 : 6;
-  return m > most ? most : m;
+  const int32_t m = (int32_t)((64 * 1024) / per_token);
+  return m > 8 ? 8 : m;
+}
+
+// The GEMM's block for a few tokens takes 16 rows through K stage by stage, which no other block of the CU hides: up to
+// 4096 rows 2.6 us and 1.05 ns a value of K (int6 1.2, bias 0 3.2), whatever the rows. The GEMV's time goes with the tokens
+// and with its blocks of four rows a CU (q), and falls only slightly with K, so it is the faster one for few rows, few
+// tokens and long rows. Measured, us a launch (each launch its own weights) here / in the GEMM:
+//   bias 64, int8: 1024 rows of 4096, 2 tokens 4.9 / 7.4, 7 tokens 6.7 / 7.5; of 512, 4 tokens 3.4 / 3.3; 512 rows of 14336,
+//     7 tokens 15.8 / 17.7, 8 tokens 19.0 / 17.7; 2048 rows of 4096, 6 tokens 7.1 / 7.6, 8 tokens 8.2 / 7.5; of 1024, 4 tokens
+//     4.8 / 4.4; of 14336, 5 tokens 17.3 / 18.3, 6 tokens 19.4 / 18.3; 3072 rows of 4096, 4 tokens slower, of 8192, 2 tokens
+//     faster; 4096 rows of 4096, 2 tokens 10.7 / 8.4;
+//   bias 64, int6 (fewer bytes a row): 1024 rows of 14336, 2 tokens 8.5 / 19.9, 8 tokens 16.3 / 20.0; of 512, 4 tokens 3.9 / 3.3;
+//     2048 rows of 4096, 8 tokens 7.2 / 8.1; of 1024, 4 tokens 5.9 / 4.7; 4096 rows of 14336, 2 tokens 18.1 / 20.3, 3 tokens
+//     21.7 / 20.3;
+//   bias 0 (four sums a group): 1024 rows of 4096, 7 tokens (one pass) 8.2 / 16.4, int6 6.0 / 16.6; 96 rows of 14336 in
+//     passes of 2, 7 tokens 44.4 / 48.1; 1536 rows of 6144, 10 tokens (two passes) int6 16.9 / 23.1; 8192 rows of 4096,
+//     7 tokens 33.5 / 21.0; 1024 rows of 3072, 14 tokens slower, int6 11.2 / 13.3.
+bool gemv_faster(int32_t rows, int32_t k, int32_t m, bool six, bool relaxed) {
+  if (m == 1) return true;
+  const int32_t step = gemv_tokens(k, relaxed), q = (rows - 1) / 1024 + 1;  // four-row blocks a CU of 256
+  if (step < 1) return false;
+  const int32_t passes = (m + step - 1) / step;
+  if (relaxed) {
+    struct Line {
+      int32_t k, m;  // the shortest rows, the most tokens
+    };
+    const Line int8[4] = {{600, k > 8192 ? 7 : 8}, {1800, k > 8192 ? 5 : 6}, {7000, 3}, {INT32_MAX, 0}};
+    const Line int6[4] = {{850, 8}, {2048, k > 16384 ? 6 : 8}, {7000, 3}, {12000, 2}};
+    if (q > 4 || passes > 1) return false;
+    const Line line = six ? int6[q - 1] : int8[q - 1];
+    return k >= line.k && m <= line.m;
+  }
+  if (m <= 6 && passes == 1) return true;
+  const int32_t most = six ? 16 : 12;
+  if (q > 4) return false;
+  if (step == 8) {  // (rows of up to 3.9 KiB)
+    return m <= 8 ? k >= (q < 4 ? 320 * q : 2048) : q == 1 && k >= 2048 && m <= most;
+  }
+  return m <= most && passes <= std::max(step > 3 ? 1 : 2, (step > 3 ? 4 : (six && step == 3 ? 8 : 7) - step) - q);
 }
 
 bool decode_takes_f32(int32_t k, bool six, bool relaxed) {
@@ -1042,7 +1074,21 @@ hipError_t launch_gemv(const MatArgs &a, bool six, bool relaxed, hipStream_t s) 
   if (a.persistent) return launch_persistent(a, s);
   if (!sums && !six && relaxed && a.m == 1 && a.k <= 20 * 1024) return launch_decode(a, s);
   if (!sums && six && relaxed && a.m == 1 && a.k <= 24 * 1024 && (a.k / GS) % 2 == 0) return launch_decode6(a, s);
-  if (!sums && a.m > gemv_tokens(a.k, relaxed)) return hipErrorInvalidValue;
+  const int32_t step = sums ? 8 : gemv_tokens(a.k, relaxed);
+  if (step < 1 || a.m < 1) return hipErrorInvalidValue;
+  if (a.m > step) {  // in passes
+    if (sums) return hipErrorInvalidValue;
+    for (int32_t t0 = 0; t0 < a.m; t0 += step) {
+      MatArgs p = a;
+      p.m = std::min(step, a.m - t0);
+      p.xq = a.xq + (int64_t)t0 * a.xq_stride;
+      p.xs = a.xs + (int64_t)t0 * a.xs_stride;
+      for (int i = 0; i < a.nseg; ++i) p.seg[i].y = a.seg[i].y + (int64_t)t0 * a.seg[i].y_stride;
+      const hipError_t e = launch_gemv(p, six, relaxed, s);
+      if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
+  }
   if (six) {
     if (relaxed) return sums ? launch_sel<true, true, true>(a, s) : launch_sel<true, true, false>(a, s);
     return sums ? launch_sel<true, false, true>(a, s) : launch_sel<true, false, false>(a, s);

@@ -91,8 +91,8 @@ struct MatArgs {
 // the launch goes another way
 int32_t decode_block_rows(int32_t k, int32_t total_rows, bool six, bool relaxed, bool xf, bool qkv_on);
 
-// decode GEMV: exact int32 group sums, the reference's float32 order; bias 64 one token, bias 0 up to 6 (m <=
-// gemv_tokens()), with a.sums up to 8
+// decode GEMV: exact int32 group sums, the reference's float32 order; more than gemv_tokens() tokens in passes, one launch
+// after another (a.sums: up to 8 tokens)
 hipError_t launch_gemv(const MatArgs &a, bool six, bool relaxed, hipStream_t s);
 // whether a one-token launch_gemv of rows of k takes its activations as float32 (MatArgs.xf)
 bool decode_takes_f32(int32_t k, bool six, bool relaxed);
@@ -100,9 +100,10 @@ bool decode_takes_f32(int32_t k, bool six, bool relaxed);
 bool decode_persistent(int32_t k, bool six, bool relaxed);
 // whether a one-token launch_gemv of rows of k finishes q / k / v itself (MatArgs.qkv)
 bool decode_fuses_qkv(int32_t k, bool six, bool relaxed);
-// the most tokens one launch_gemv takes for rows of k, 0 where a row's products pass the block's LDS; more tokens go to
-// launch_gemm
+// the most tokens one launch of launch_gemv takes for rows of k, 0 where a row's products pass the block's LDS
 int32_t gemv_tokens(int32_t k, bool relaxed);
+// whether launch_gemv takes m tokens against `rows` rows of k in less time than launch_gemm (one token: always)
+bool gemv_faster(int32_t rows, int32_t k, int32_t m, bool six, bool relaxed);
 // GEMM on i8 MFMA, any m: the same bits as launch_gemv per (token, row); with a.sums (one segment, bias 64) the exact
 // int32 group sums [m][rows][K/32] instead
 hipError_t launch_gemm(const MatArgs &a, bool six, bool relaxed, hipStream_t s);
