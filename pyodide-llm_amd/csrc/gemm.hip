@@ -212,7 +212,7 @@ __device__ __forceinline__ void glu_epilogue(const MatArgs &a, float (&out)[2][1
 // with SUMS the kernel writes the exact int32 group sums S_g to a.sums [m][rows][G] instead (one segment); with GLU
 // the SwiGLU's quantized output (glu_epilogue)
 // (two waves a SIMD: the register budget that keeps the MFMA results in VGPRs, no AGPR copies)
-template <bool SIX, bool SUMS, bool GLU>
+template <bool SIX, bool SUMS, bool GLU, bool BIAS = false>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2))) void gemm_kernel(const MatArgs a) {
   __shared__ Stage stage[2];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -320,8 +320,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2))) void ge
     glu_epilogue(a, out, reinterpret_cast<float *>(&stage[0]), r0, t0, wave, lane);
     return;
   }
-  // y[t][r] = out (or y + out), + bias: the lane's two tokens, its 16 rows in 4 runs of 4
-  const bool biased = a.seg[0].bias || a.seg[1].bias || a.seg[2].bias;  // (uniform: most launches have none)
+  // y[t][r] = out (or y + out), with BIAS + bias: the lane's two tokens, its 16 rows in 4 runs of 4. (BIAS as a kernel of its
+  // own: under a run-time test it took 2-5% of a launch of short rows, 57,344 x 768, 200 tokens 75.6 -> 78.9 us.)
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
     const int t = t0 + wt * 64 + h * 32 + (lane & 31);
@@ -344,7 +344,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2))) void ge
       const int accumulate = (si == 2 ? a.seg[2].accumulate : si == 1 ? a.seg[1].accumulate : a.seg[0].accumulate);
       float *dst = y + (int64_t)t * stride + r;
       float o = accumulate ? *dst + out[h][v] : out[h][v];
-      if (biased) {
+      if constexpr (BIAS) {
         const float *bias = (si == 2 ? a.seg[2].bias : si == 1 ? a.seg[1].bias : a.seg[0].bias);
         if (bias) o = o + bias[r];
       }
@@ -368,6 +368,11 @@ hipError_t launch_gemm(const MatArgs &a, bool six, bool relaxed, hipStream_t s) 
       gemm_kernel<true, true, false><<<grid, NT, 0, s>>>(a);
     else
       gemm_kernel<false, true, false><<<grid, NT, 0, s>>>(a);
+  } else if (a.seg[0].bias || a.seg[1].bias || a.seg[2].bias) {
+    if (six)
+      gemm_kernel<true, false, false, true><<<grid, NT, 0, s>>>(a);
+    else
+      gemm_kernel<false, false, false, true><<<grid, NT, 0, s>>>(a);
   } else {
     if (six)
       gemm_kernel<true, false, false><<<grid, NT, 0, s>>>(a);

@@ -78,3 +78,24 @@ def test_layer_norm_forms_epilogues(arch, m):
     assert same_bits(kv["keys"], k.reshape(-1)) and same_bits(kv["values"], v.reshape(-1))
     eng.release()
     ref.close()
+
+
+@pytest.mark.parametrize("six", [0, 1])
+def test_biases_of_full_grids(six):
+    """GPT-2's wo and w2 with a residual add and a bias where the 64 x 128 blocks take them (4096 rows, 1024 tokens)"""
+    cfg = ol.config(dim=4096, hidden_dim=256, n_layers=2, n_heads=16, n_kv_heads=16, head_size=256, vocab_size=64,
+                    seq_len=1024, shared_classifier=1, half_kv=1, arch="gpt2", six=six)
+    tensors, size = ol.places(cfg)
+    ck = ol.vary_vectors(cfg, tensors, ol.synth_checkpoint(cfg, tensors, size, seed=8), seed=9)
+    cos, sin = package().rope_tables(cfg.seq_len, cfg.head_size, 10000.0, cfg.rotary)
+    tokens = [int(t) for t in np.random.default_rng(six).integers(0, cfg.vocab_size, size=1024)]
+    ref = ol.Model(cfg, tensors, ck, cos, sin, max_block=1024)
+    eng = package().open_config(cfg, tensors, ck, cos, sin, max_block=1024)
+    ref.run(tokens, 0, False)
+    eng.forwardMany(tokens, 0)
+    kv, (k, v) = eng.keysAndValues(1020, 4), ref.kv(1020, 4)
+    assert same_bits(kv["keys"], k.reshape(-1)) and same_bits(kv["values"], v.reshape(-1))
+    kv, (k, v) = eng.keysAndValues(0, 600), ref.kv(0, 600)
+    assert same_bits(kv["keys"], k.reshape(-1)) and same_bits(kv["values"], v.reshape(-1))
+    eng.release()
+    ref.close()
