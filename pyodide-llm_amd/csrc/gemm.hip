@@ -359,7 +359,8 @@ hipError_t launch_gemm(const MatArgs &a, bool six, bool relaxed, hipStream_t s) 
   if (a.m < 1 || a.total_rows < 1 || a.k < 32 || a.k % 32) return hipErrorInvalidValue;
   if (a.sums && (a.nseg != 1 || !relaxed)) return hipErrorInvalidValue;
   if (a.qkv.on && (a.sums || a.nseg != 3 || !gemm_finishes(a.total_rows, a.m, relaxed))) return hipErrorInvalidValue;
-  if (!a.sums && (!relaxed || gemm_chains_faster(a.total_rows, a.m, false))) return launch_gemm_chains(a, six, relaxed, s);
+  if (!a.sums && (!relaxed || a.qkv.on || gemm_chains_faster(a.total_rows, a.m, a.k, false)))
+    return launch_gemm_chains(a, six, relaxed, s);
   const int64_t blocks = (int64_t)((a.total_rows + BR - 1) / BR) * ((a.m + BT - 1) / BT);
   if (blocks > (1ll << 30)) return hipErrorInvalidValue;
   const dim3 grid((unsigned)blocks);
@@ -382,7 +383,8 @@ hipError_t launch_gemm(const MatArgs &a, bool six, bool relaxed, hipStream_t s) 
   return hipGetLastError();
 }
 
-bool gemm_finishes(int32_t rows, int32_t m, bool relaxed) { return !relaxed || gemm_chains_faster(rows, m, false); }
+// (the line of long rows for every K: an epilogue saves a launch)
+bool gemm_finishes(int32_t rows, int32_t m, bool relaxed) { return !relaxed || gemm_chains_faster(rows, m, INT32_MAX, false); }
 
 // a quantized output of `hidden` units: its 4-byte runs and its scales aligned and inside [m][q_stride] / [m][s_stride]
 static bool takes_units(const GluOut &g, int32_t hidden) {
@@ -401,7 +403,7 @@ hipError_t launch_gemm_glu(const MatArgs &a, bool six, bool relaxed, hipStream_t
   if (a.m < 1 || a.nseg != 2 || a.sums || a.k < 32 || a.k % 32) return hipErrorInvalidValue;
   const int hidden = a.seg[0].rows;
   if (!takes_units(a.glu, hidden) || a.seg[1].rows != hidden || a.total_rows != 2 * hidden) return hipErrorInvalidValue;
-  if (!relaxed || gemm_chains_faster(a.total_rows, a.m, true)) return launch_gemm_chains_glu(a, six, relaxed, s);
+  if (!relaxed || gemm_chains_faster(a.total_rows, a.m, a.k, true)) return launch_gemm_chains_glu(a, six, relaxed, s);
   const int64_t blocks = (int64_t)(hidden / 32) * ((a.m + BT - 1) / BT);
   if (blocks > (1ll << 30)) return hipErrorInvalidValue;
   if (six)

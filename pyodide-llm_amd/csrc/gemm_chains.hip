@@ -525,11 +525,16 @@ hipError_t launch_gelu_tile(const MatArgs &a, hipStream_t s) {
 // 46.9 / 60.4, 1024 tokens 92.4 / 76.0; 6144 x 4096, 384 tokens 57.0 / 66.5, 512 tokens 69.4 / 67.4; 14336 x 4096, 100
 // tokens 48.5 / 59.9, 200 tokens 78.7 / 72.7, 300 tokens (a second round there) 101.9 / 124.2; the SwiGLU at 28672 x
 // 4096, 64 tokens 57.0 / 65.6, 96 tokens 73.6 / 66.9, at 4096 x 512, 300 tokens 11.3 / 12.1, 511 tokens 14.1 / 12.3.
-bool gemm_chains_faster(int32_t rows, int32_t m, bool glu) {
+// Short rows leave the blocks' hand-over and stores, which weigh more on blocks of 64 x 32 (us there / here): K of 96, 14336
+// rows, 100 tokens (one of theirs a CU, 896 of these) 9.3 / 11.0, 4096 rows, 256 tokens (512) 8.8 / 7.3; K of 192, 14336 rows,
+// 100 tokens 11.5 / 12.0, 6144 rows, 400 tokens (1248 in a round) 16.2 / 14.0; K of 320, 28672 rows, 400 tokens (1456 a round)
+// 54.8 / 58.3, 6144 rows, 400 tokens 18.2 / 16.4; K of 512, 28672 rows, 400 tokens 64.4 / 59.1.
+bool gemm_chains_faster(int32_t rows, int32_t m, int32_t k, bool glu) {
   const int64_t theirs = tiles(rows, 64) * tiles(m, 128), ours = tiles(rows, 64) * tiles(m, 32);
   const int64_t rounds = tiles(theirs, 2 * CUS);
   if (glu) return ours <= (theirs <= CUS ? 720 : 1000 * rounds);
-  return ours <= (theirs <= CUS ? 1250 : 1480 * rounds);
+  if (theirs <= CUS) return ours <= (k < 512 ? std::max(512, std::min(1250, 440 + 2 * k)) : 1250);
+  return ours <= (k < 512 ? 1400 : 1480) * rounds;
 }
 
 hipError_t launch_gemm_chains(const MatArgs &a, bool six, bool relaxed, hipStream_t s) {

@@ -116,7 +116,7 @@ hipError_t launch_gemm_gelu(const MatArgs &a, bool six, bool relaxed, hipStream_
 bool gemm_finishes(int32_t rows, int32_t m, bool relaxed);
 // gemm_chains.hip: the GEMM with each float32 lane chain on a wave of its own, for bias 0 and for the grids where it is
 // the faster one (rows: of every segment). launch_gemm and launch_gemm_glu check the arguments and choose.
-bool gemm_chains_faster(int32_t rows, int32_t m, bool glu);
+bool gemm_chains_faster(int32_t rows, int32_t m, int32_t k, bool glu);
 hipError_t launch_gemm_chains(const MatArgs &a, bool six, bool relaxed, hipStream_t s);
 hipError_t launch_gemm_chains_glu(const MatArgs &a, bool six, bool relaxed, hipStream_t s);
 hipError_t launch_gemm_chains_gelu(const MatArgs &a, bool six, bool relaxed, hipStream_t s);

@@ -28,6 +28,16 @@ def test_matmul_bits(rows, k, m, six, bias):
     assert same_bits(gl.matmul(xq, xs, w, ws, rows, k, bias, six), ol.matmul(xq, xs, w, ws, rows, k, bias, six))
 
 
+# rows shorter than 512 leave the chains' blocks for the 64 x 128 ones earlier: of 96 values 429 blocks stay and 680 do not, of
+# 32 495 stay; past one of those a CU 1469 blocks of 512 values stay, and of 480 do not
+@pytest.mark.parametrize("six", [0, 1])
+@pytest.mark.parametrize("rows,k,m", [(2112, 96, 416), (2176, 96, 640), (2112, 32, 480), (7232, 480, 416), (7232, 512, 416)])
+def test_short_rows(rows, k, m, six):
+    w, ws = weights(rows, k, six)
+    xq, xs = activations(m, k, 64)
+    assert same_bits(gl.matmul(xq, xs, w, ws, rows, k, 64, six), ol.matmul(xq, xs, w, ws, rows, k, 64, six))
+
+
 @pytest.mark.parametrize("m", [2, 6, 7, 8, 9])
 def test_where_the_gemv_ends(m):
     """bias 0: up to 6 tokens on the GEMV (2 where a row's products are long), more on the GEMM"""
@@ -96,6 +106,24 @@ def test_biases_of_full_grids(six):
     kv, (k, v) = eng.keysAndValues(1020, 4), ref.kv(1020, 4)
     assert same_bits(kv["keys"], k.reshape(-1)) and same_bits(kv["values"], v.reshape(-1))
     kv, (k, v) = eng.keysAndValues(0, 600), ref.kv(0, 600)
+    assert same_bits(kv["keys"], k.reshape(-1)) and same_bits(kv["values"], v.reshape(-1))
+    eng.release()
+    ref.close()
+
+
+def test_short_rows_finish_qkv():
+    """q/k/v of a pass whose rows are so short that a plain matmul would leave the chains' blocks: the epilogue keeps them"""
+    cfg = ol.config(dim=96, hidden_dim=96, n_layers=2, n_heads=32, n_kv_heads=32, head_size=64, vocab_size=64, seq_len=256,
+                    shared_classifier=1)
+    tensors, size = ol.places(cfg)
+    ck = ol.vary_vectors(cfg, tensors, ol.synth_checkpoint(cfg, tensors, size, seed=8), seed=9)
+    cos, sin = package().rope_tables(cfg.seq_len, cfg.head_size, 10000.0)
+    tokens = [int(t) for t in np.random.default_rng(1).integers(0, cfg.vocab_size, size=256)]
+    ref = ol.Model(cfg, tensors, ck, cos, sin, max_block=256)
+    eng = package().open_config(cfg, tensors, ck, cos, sin, max_block=256)
+    ref.run(tokens, 0, False)
+    eng.forwardMany(tokens, 0)
+    kv, (k, v) = eng.keysAndValues(0, 256), ref.kv(0, 256)
     assert same_bits(kv["keys"], k.reshape(-1)) and same_bits(kv["values"], v.reshape(-1))
     eng.release()
     ref.close()
