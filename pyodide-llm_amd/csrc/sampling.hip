@@ -228,16 +228,31 @@ __device__ __forceinline__ double add_values(const float (&v)[SEG], double acc) 
 
 // One chunk (values b.., lane L's 32 at b + 32 L) exactly from run, by one wave: the lanes in parallel while the sum
 // stays in one binade; a lane that takes it out of its binade adds its values one after another; then the lanes after
-// it in parallel again. After two such lanes (a sum that still crosses binades often: a parallel pass costs about as
-// much as twenty lanes' adds in turn), and from a sum of 0, the rest of the chunk goes lane by lane. Returns the
-// chunk's end (every lane); with cp, the checkpoints of the chunk's values. (A nucleus draw's total of 1091 kept values,
-// one chunk from 0: 48,000 -> 13,400 cycles with the turns past the last value left out, no parallel pass from 0, and the
-// conversions out of the chain.)
+// it in parallel again. After two such lanes (a sum that still crosses binades often) the rest of the chunk goes lane by
+// lane. A parallel pass costs about as much as 48 lanes' adds in turn (PASS_TURNS), so from a sum of 0 the lanes go in turn
+// from the start, unless the first lane's sum puts the next crossing further than that (a likely token among the first 32
+// values): then that lane, one pass, and the rest in turn. Returns the chunk's end (every lane); with cp, the checkpoints
+// of the chunk's values. (A nucleus draw's total of 1091 kept values, one chunk from 0: 48,000 -> 13,400 cycles with the
+// turns past the last value left out, no parallel pass and the conversions out of the chain; a whole chunk behind a likely
+// token, in a draw of 32,000 logits: 44.3 us in turn, 41.7 with the pass.)
+constexpr int PASS_TURNS = 48;
+__device__ __forceinline__ double lane_in_order(const float (&v)[SEG], double run, int from, double &pre);
 __device__ __forceinline__ double chunk_exact(const float (&v)[SEG], double run, int b, int count, double *cp) {
-  const int lane = threadIdx.x & 63;
+  const int lane = threadIdx.x & 63, lanes = min(64, (count - b + SEG - 1) / SEG);
   double pre = 0.0;  // this lane's sum before its values
-  int from = 0;
-  for (int crossed = 0; run > 0.0 && from < 64 && crossed < 2; ++crossed) {
+  int from = 0, crossed = 0;
+  if (!(run > 0.0) && lanes > PASS_TURNS) {
+    float t = 0.0f;  // (the lanes' sums in any order: they only guess where the sum crosses)
+#pragma unroll
+    for (int u = 0; u < SEG; ++u) t += v[u];
+    const double upto = lanes_upto((double)t), first = from_lane(upto, 0);
+    const uint64_t past = __ballot(upto >= __builtin_ldexp(1.0, binade(first) + 1));
+    if (first > 0.0 && (past ? __builtin_ctzll(past) : 64) > PASS_TURNS) {
+      run = lane_in_order(v, run, 0, pre);
+      from = crossed = 1;
+    }
+  }
+  for (; run > 0.0 && from < 64 && crossed < 2; ++crossed) {
     double start = run, end = 0.0;
     const int cross = chunk_lanes(v, run, from, &start, &end);
     if (lane >= from && lane <= cross) pre = start;
@@ -253,7 +268,6 @@ __device__ __forceinline__ double chunk_exact(const float (&v)[SEG], double run,
   }
   // lane by lane: in turn s lane s adds its values to the sum the lane below handed it (every lane adds its own, all
   // widened before the first turn), up to the last lane with a value of the chunk (+0.0 past it changes no sum)
-  const int lanes = min(64, (count - b + SEG - 1) / SEG);
   if (from < lanes) {
     double d[SEG], acc = run;
 #pragma unroll
