@@ -608,13 +608,21 @@ __global__ __launch_bounds__(A3_NT) void attend3_kernel(const AttnArgs a, const 
 
 // The whole of a decode attention in one launch, for contexts of up to A1_MOST positions: one block of 1024 threads a
 // (token, query head, 16 columns), as attend2_kernel, that makes the head's scores itself, a thread a position. The head's
-// other column blocks repeat them (A1_SCORES bounds the keys a block reads), which costs less than the scores' launch
+// other column blocks repeat them (a1_scores bounds the keys a block reads), which costs less than the scores' launch
 // where everything fits the caches. Then the maximum over the block, and attend2_kernel's steps with a thread a
 // (four-position block, 4 columns), its values requested with the keys. Bound by latency: the loads, two ordered sums of
 // count / 4 steps, five barriers. (With the FFN's activation in w2's GEMV: two launches a layer fewer; a sampled step of
 // the 15M shape 230 -> 203 us.)
-constexpr int A1_MOST = 1024;          // positions: one a thread, four threads a four-position block
-constexpr int A1_SCORES = 64 * 1024;   // positions * head size at most
+constexpr int A1_MOST = 1024;  // positions: one a thread, four threads a four-position block
+// Positions * head size at most: a replayed step's launch is fixed by the model's whole context, so the line lies where a
+// step's mean over the positions of the context meets that of scores_kernel + attend2_kernel. A replayed layer of 512
+// dims, us here / with the two launches, at 3%, 50% and 97% of the context, and the mean over it:
+//   64 Ki: 8 heads of 64, 1024 positions, float16 23.4 / 27.3, 28.8 / 28.0, 32.1 / 30.1, mean 28.1 / 28.3; float32 22.2 / 26.1,
+//     29.3 / 29.0, 33.3 / 29.9, mean 28.6 / 28.4; 12 heads 28.3 / 29.7 and 29.1 / 29.4; 32 / 8 heads of 128, 512 positions,
+//     float32 30.9 / 32.2; 8 / 4 heads of 256, 256 positions 29.3 / 31.7; 32 heads of 96, 680 positions, float16 31.4 / 33.0,
+//     float32 (two loads of 48 dims a position) 27.2 / 31.4, 32.2 / 32.2, 38.8 / 33.3, mean 32.6 / 32.3: there 48 Ki, 31.0 / 31.8;
+//   48 Ki: 6 heads of 48, 1024 positions, float16 25.7 / 27.7, float32 26.8 / 27.4; 16 Ki: 8 heads of 16 23.1 / 25.9.
+constexpr int a1_scores(int hs, bool half) { return (hs == 96 && !half ? 48 : 64) * 1024; }
 
 template <int HS> constexpr int a1_chunk() { return HS <= 64 ? HS : (HS % 64 == 0 ? 64 : 48); }  // dims in registers
 
@@ -716,7 +724,7 @@ __global__ __launch_bounds__(A2_NT) void attend1_kernel(const AttnArgs a) {
 // whether attend1_kernel takes a decode launch
 bool attend1_takes(const AttnArgs &a) {
   const int count = a.pos0 + a.m;
-  return a.hs % A2_AC == 0 && count <= A1_MOST && count * a.hs <= A1_SCORES;
+  return a.hs % A2_AC == 0 && count <= A1_MOST && count * a.hs <= a1_scores(a.hs, a.half);
 }
 
 // LDS bytes of attend_kernel for the largest count of a launch (ring slots into *nslot), 0 where it does not fit

@@ -234,7 +234,7 @@ __device__ __forceinline__ double add_values(const float (&v)[SEG], double acc) 
 // values): then that lane, one pass, and the rest in turn. Returns the chunk's end (every lane); with cp, the checkpoints
 // of the chunk's values. (A nucleus draw's total of 1091 kept values, one chunk from 0: 48,000 -> 13,400 cycles with the
 // turns past the last value left out, no parallel pass and the conversions out of the chain; a whole chunk behind a likely
-// token, in a draw of 32,000 logits: 44.3 us in turn, 41.7 with the pass.)
+// token, in a draw of 32,000 logits: 44.3 us in turn, 39.8 with the pass.)
 constexpr int PASS_TURNS = 48;
 __device__ __forceinline__ double lane_in_order(const float (&v)[SEG], double run, int from, double &pre);
 __device__ __forceinline__ double chunk_exact(const float (&v)[SEG], double run, int b, int count, double *cp) {

@@ -37,7 +37,8 @@ def steps(cfg, prompt, count, seed):
     (48, 4, 4, 0, 9),        # the first positions: no whole four, a tail of every length
     (16, 8, 2, 253, 8),      # across a wave's positions and a four's thread
     (64, 4, 1, 1020, 8),     # the last positions of the one launch and the first past it
-    (96, 2, 2, 680, 6),      # the keys' bound: 682 positions of 96
+    (96, 2, 2, 680, 6),      # the keys' bound: 682 positions of 96 in float16
+    (96, 2, 2, 509, 6),      # and 512 in float32
     (128, 4, 2, 509, 6),     # 512 of 128
     (256, 1, 1, 253, 6),     # 256 of 256
 ])
