@@ -1097,7 +1097,7 @@ int32_t he_generate_many(he_engine *e, int32_t token, int32_t pos, const int32_t
   // tokens are read once at its end, and the first step that ends the call (a stop token, a declined draw, a largest
   // logit that is not finite) is known from state[STATE_HALTED]; the round's replays after it are spent for nothing
   // (their cache rows lie past the call's positions, rewritten by whatever step takes those positions next), its
-  // logits kept apart for he_logits. Rounds are shorter where stop tokens may end the call.
+  // logits kept apart for he_logits where replays came after it. Rounds are shorter where stop tokens may end the call.
   RunParams &hp = *e->host_params;
   hp.temperature = temperature;
   hp.topp = topp;
@@ -1114,6 +1114,7 @@ int32_t he_generate_many(he_engine *e, int32_t token, int32_t pos, const int32_t
   for (bool first = true; done < count; first = false) {
     const int32_t n = std::min(round, count - done);
     for (int32_t i = 0; i < RUN_RANDOMS; ++i) hp.randoms[i] = temperature > 0.0f && i < n ? randoms[done + i] : 0.0;
+    hp.steps = n;
     hs[STATE_WORDS] = token;
     hs[STATE_POS] = pos + done;
     hs[STATE_STEP] = 0;
@@ -1134,7 +1135,7 @@ int32_t he_generate_many(he_engine *e, int32_t token, int32_t pos, const int32_t
     for (int32_t j = 0; j < (halted ? halted : n); ++j) {
       const int32_t id = e->host_ids[j];
       if (halted && j == halted - 1) {
-        e->logits_kept = true;
+        e->logits_kept = halted < n;  // (no replay came after the round's last step)
         if (id == SAMPLE_NOT_FINITE || !std::isfinite(e->host_values[j]))
           return fail(HE_E_NOTFINITE, "the largest logit is not finite");
         if (id != SAMPLE_DECLINED) ids[(*n_ids)++] = id;  // the stop token, last

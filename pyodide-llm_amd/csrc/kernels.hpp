@@ -210,8 +210,8 @@ hipError_t launch_mfma_ceiling(int32_t passes, int32_t first, int32_t times, int
                                hipStream_t s);
 struct RunParams;
 // the end of a replayed step, by the launch that chooses its token (stepend.hpp): where this step ends the call (a stop
-// token, no token, a largest logit that is not finite) and none before it did, its logits into kept and
-// state[STATE_HALTED] = step + 1; its token and value into ids / values at the step, the token into the window and as the
+// token, no token, a largest logit that is not finite) and none before it did, state[STATE_HALTED] = step + 1, and its logits
+// into kept unless it is the round's last step; its token and value into ids / values at the step, the token into the window and as the
 // next step's input (tokens[0]), the position and the step advanced. params null: no step to end.
 struct StepEnd {
   const float *logits;
@@ -285,6 +285,7 @@ struct RunParams {
   float temperature, topp, penalty;
   int32_t n_stops;
   int32_t stops[RUN_STOPS_MOST];
+  int32_t steps;                // the round's steps
 };
 // a step's draw (as launch_sample) with the call's temperature and top-p and the round's random number of the step;
 // with window, the call's penalty over the window's state[STATE_WINDOW] tokens first (launch_penalize_steps's, in the

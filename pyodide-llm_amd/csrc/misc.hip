@@ -363,7 +363,7 @@ __global__ __launch_bounds__(256) void argmax_stage(float *ov, int32_t *oi, cons
     ov[blockIdx.x] = sv[0];
     oi[blockIdx.x] = si[0];
   }
-  if (end.params) step_end(end, si[0], sv[0], threadIdx.x, 256);
+  if (end.params) step_end<16>(end, si[0], sv[0], threadIdx.x, 256);
 }
 
 // ---- the device twin of the oracle's synthetic checkpoint (oracle/oracle.c or_synth_value, or_quantize,

@@ -1072,7 +1072,7 @@ __global__ __launch_bounds__(ST) void draw_kernel(int32_t n, const DrawParts *pa
     *out_token = token;
     *out_best = best;
   }
-  if (end.params) step_end(end, token, best, threadIdx.x, ST);
+  if (end.params) step_end<8>(end, token, best, threadIdx.x, ST);
 }
 
 // the five launches of a draw (the settings as values, or with params the call's and the step's from device memory;
