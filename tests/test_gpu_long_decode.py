@@ -59,7 +59,7 @@ def test_replayed_steps_of_a_long_context(heads, kv_heads, head_size, half_kv):
 
 @pytest.mark.parametrize("half_kv", [0, 1])
 def test_replayed_steps_of_the_longest_context(half_kv):
-    replayed_steps(2, 1, 16, half_kv, 32768, LONGEST)
+    replayed_steps(4, 2, 16, half_kv, 32768, LONGEST)
 
 
 def replayed_steps(heads, kv_heads, head_size, half_kv, seq_len, counts):
