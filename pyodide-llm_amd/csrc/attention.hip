@@ -9,9 +9,9 @@
 // The keys lie as the positions' rows ([seq_len][kv_dim]), the values as the columns' runs of positions
 // ([kv_dim][vstride]). Launches: (A) the scores of 64-position tiles, every CU streaming keys once for the nh / nkv
 // query heads that share them, with each tile's maxima; then for a few tokens (decode) one launch (B + C) a
-// (token, head, 16 or 32 columns): the exponentials, their ordered sum, and the weighted values. A prompt block's
-// scores, and the separate softmax and weighted values of prompt blocks and of contexts past these kernels' LDS, are
-// attention_tokens.hip's.
+// (token, head, 16 or 32 columns): the exponentials, their ordered sum, and the weighted values (short contexts: the
+// scores too, attend1_kernel). A prompt block's scores, and the separate softmax and weighted values of prompt blocks
+// and of contexts past these kernels' LDS, are attention_tokens.hip's.
 #pragma clang fp contract(off)
 
 #include <algorithm>

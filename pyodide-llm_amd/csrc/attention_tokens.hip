@@ -23,21 +23,6 @@ namespace {
 // add a product instead of a multiply and an add. The head is staged in chunks of DC dims (the rows' queries and the
 // tile's keys, double buffered in LDS: the next chunk's loads in flight while this one is summed). No tile maxima:
 // the softmax takes each row's largest score from the scores themselves.
-// The blocks of the prompt's kernels by XCD: block b runs on XCD b % 8, and the (kv head, token block, x) triples, x
-// fastest, are dealt to the XCDs in 8 contiguous ranges, so that what the blocks of a kv head share (its keys and
-// values, the score rows that one kernel writes and the next reads) stays in one XCD's L2. A kv head's token blocks come
-// from both ends in turn: the later ones see more positions, and where a kv head's blocks are cut between two XCDs both
-// get short and long ones.
-struct TokenBlock {
-  int x, kh, z;
-};
-__device__ __forceinline__ TokenBlock token_block(int nx, int nz) {
-  const int n = gridDim.x, xcd = blockIdx.x & 7;
-  const int idx = xcd * (n / 8) + min(xcd, n % 8) + (blockIdx.x >> 3);
-  const int rest = idx / nx, zi = rest % nz;
-  return {idx % nx, rest / nz, (zi & 1) ? nz - 1 - zi / 2 : zi / 2};
-}
-
 template <int HS> constexpr int score_chunk() { return HS % 32 == 0 ? 32 : 16; }
 constexpr int SCORE_ROWS = 64;  // (token, head) rows a block
 
@@ -444,6 +429,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void p
     __syncthreads();
     quantize_rows<HS, R>(a, rows, C + 4, kh, j0, t0, tt_n, mul, tid);
   }
+}
+
+// (C')'s blocks by XCD: block b runs on XCD b % 8, and the (kv head, token block, x) triples, x fastest, are dealt to the
+// XCDs in 8 contiguous ranges, so that what the blocks of a kv head share (its values, and a row's weights for every x)
+// stays in one XCD's L2. A kv head's token blocks come from both ends in turn: the later ones see more positions, and
+// where a kv head's blocks are cut between two XCDs both get short and long ones.
+struct TokenBlock {
+  int x, kh, z;
+};
+__device__ __forceinline__ TokenBlock token_block(int nx, int nz) {
+  const int n = gridDim.x, xcd = blockIdx.x & 7;
+  const int idx = xcd * (n / 8) + min(xcd, n % 8) + (blockIdx.x >> 3);
+  const int rest = idx / nx, zi = rest % nz;
+  return {idx % nx, rest / nz, (zi & 1) ? nz - 1 - zi / 2 : zi / 2};
 }
 
 // (C') for grids too small to fill the chip with (C)'s one wave a tile: four waves share one tile of 16 (token, head) rows

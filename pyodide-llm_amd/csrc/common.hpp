@@ -13,9 +13,8 @@ namespace ple {
 
 // ---- integer helpers ----
 
-// i32.trunc_sat_f32_s: NaN to 0, out of range to the nearest end (the conversion of quantize_x, kernels/kernel.ts:145)
-// (as selects: the clamped conversion, then the top end and NaN)
-// (the conversion instruction's own results)
+// i32.trunc_sat_f32_s: NaN to 0, out of range to the nearest end (the conversion of quantize_x, kernels/kernel.ts:145):
+// what the conversion instruction gives
 __device__ __forceinline__ int32_t trunc_sat(float f) {
   int32_t i;
   asm("v_cvt_i32_f32 %0, %1" : "=v"(i) : "v"(f));
@@ -157,8 +156,8 @@ __host__ __device__ constexpr int chain_rowstride(int q4) { return ((q4 + 63) & 
 // acc + c[0] + c[1] + ... + c[n-1] in order (every add rounded), the values read from LDS 64 at a time: the second
 // 32's reads fly while the first 32 are added. (No reads carried across iterations: a loop-carried set of registers
 // makes the compiler copy it every iteration, which costs more than the latency it hides.) c 16-byte aligned.
-template <int H = 8>
-__device__ __forceinline__ float lds_chain_h(const float *c, int n, float acc) {
+__device__ __forceinline__ float lds_chain(const float *c, int n, float acc) {
+  constexpr int H = 8;
   const float4 *c4 = reinterpret_cast<const float4 *>(c);
   const int n4 = n >> 2;
   int i = 0;
@@ -206,7 +205,6 @@ __device__ __forceinline__ float lds_chain_h(const float *c, int n, float acc) {
   for (int j = n4 << 2; j < n; ++j) acc = acc + c[j];
   return acc;
 }
-__device__ __forceinline__ float lds_chain(const float *c, int n, float acc) { return lds_chain_h<8>(c, n, acc); }
 
 // Where value i of an ordered sum lies in its LDS row for chain16_registers: 32 values a segment, a segment's float4 pieces
 // turned by the segment, so that the 16 lanes' reads of one step fall on distinct banks.

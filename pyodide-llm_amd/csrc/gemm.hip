@@ -1,6 +1,7 @@
 // gemm.hip — the prefill matmul on CDNA4 i8 MFMA (bias 64): many tokens against an int8 (or int6) matrix with per-group
-// float32 scales (grids that these blocks fill; gemm_chains.hip takes the others, and bias 0), in the reference's exact float32 order (kernels/kernel_relaxed.ts:34-67 matmul_q8r and :164-183
-// matmul_q8r_tile, which is the same per (row, token); matmul_q6r :189-218 on the six.ts-widened values).
+// float32 scales (grids that these blocks fill; gemm_chains.hip takes the others, and bias 0), in the reference's exact
+// float32 order (kernels/kernel_relaxed.ts:34-67 matmul_q8r and :164-183 matmul_q8r_tile, which is the same per (row,
+// token); matmul_q6r :189-218 on the six.ts-widened values).
 //
 // For a (row r, token t): S_g = dot(w_g, q_g - 64) is an exact int32 per group g of 32. One
 // v_mfma_i32_32x32x32_i8 makes S_g for a 32-row x 32-token tile: K = 32 is exactly one group, so every MFMA output is

@@ -10,9 +10,10 @@
 // waves instead of one.
 //
 // Tiling: v_mfma_i32_16x16x32_i8 makes the exact group sums of 16 rows x 16 tokens. A wave makes RT x TT such tiles of
-// one chain; a block is RB x 4 waves (RB row parts, 4 chains) on RB * RT * 16 rows and TT * 16 tokens. A stage is CK = 8
-// groups (256 bytes of K) of the block's rows, tokens and scales in LDS, double buffered, and the loads of the stage
-// after the next are in flight in registers: two stages' loads cover the memory's latency where a CU holds one block.
+// one chain; a block is RB x 4 waves (RB row parts, 4 chains) on RB * RT * 16 rows and TT * 16 tokens. A stage is CK = 16
+// or 8 groups (512 or 256 bytes of K: launch_tile) of the block's rows, tokens and scales in LDS, double buffered, and the
+// loads of the stage after the next are in flight in registers: two stages' loads cover the memory's latency where a CU
+// holds one block.
 // For bias 0 the staging turns each half of a group's bytes so that lane sum k's 8 bytes lie side by side: the A operand
 // of chain k's wave is then the group's bytes in the lanes that hold part k and zeros in the others.
 #pragma clang fp contract(off)

@@ -40,7 +40,7 @@ def test_short_rows(rows, k, m, six):
 
 @pytest.mark.parametrize("m", [2, 6, 7, 8, 9])
 def test_where_the_gemv_ends(m):
-    """bias 0: up to 6 tokens on the GEMV (2 where a row's products are long), more on the GEMM"""
+    """bias 0, 40 rows: the GEMV in one pass, and in passes of two where a row's products are long; 9 such tokens on the GEMM"""
     for k in (96, 14336):
         w, ws = weights(40, k, 0)
         xq, xs = activations(m, k, 0)

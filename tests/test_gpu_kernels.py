@@ -99,7 +99,7 @@ def test_gemm_bits(k, rows, m, six):
 
 @pytest.mark.parametrize("six", [0, 1])
 def test_plain_order_with_many_tokens(six):
-    """bias 0 (matmul_q8's lanes) with more than 8 tokens stays on the GEMV, in passes of 8"""
+    """bias 0 (matmul_q8's lanes) with more tokens than a GEMV pass takes"""
     k, rows, m = 288, 40, 20
     w, ws = weights(rows, k, six)
     xq, xs = activations(m, k, 0)
