@@ -499,13 +499,17 @@ hipError_t launch_tile(const MatArgs &a, hipStream_t s) {
 }
 
 // the SwiGLU's blocks (32 units of w1 and of w3): 16 tokens while that is at most one block a CU (4096 rows of K 512, 64
-// tokens: 5.3 against 5.9 us; 128 tokens: 7.1 against 6.1), 48 where they hold the tokens with a tile less than two
-// blocks of 32 (28,672 rows of K 4096, 37 tokens: 46 against 52), else 32
+// tokens: 5.3 against 5.9 us; 128 tokens: 7.1 against 6.1); 48 for three tiles of tokens where the fullest CU would take
+// twice as many blocks of 32, two of which cost more than one of 48 and less than that where it would not (40 tokens, us 48 /
+// 32: 11,264 rows of K 2048, 1 or 2 a CU, 13.9 / 15.8; 16,384 of 3072, 1 or 2, 20.4 / 23.7; 28,672 of 4096, 2 or 4, 45.0 /
+// 49.8; but 22,016 of 4096, 2 or 3, 44.4 / 40.1; 37,888 of 3584, 3 or 5, 60.3 / 55.6; 57,344 of 8192, 4 or 7, 171 / 165;
+// int6 within 3% of these); else 32
 template <bool SIX, bool PLAIN>
 hipError_t launch_glu_tile(const MatArgs &a, hipStream_t s) {
   const int64_t units = tiles(a.seg[0].rows, 32), m = a.m;
   if (m <= 16 || units * tiles(m, 16) <= CUS) return launch_one<SIX, PLAIN, 2, 1, 2, 8, 2, EPI_GLU>(a, s);
-  if (tiles(m, 16) == 3) return launch_one<SIX, PLAIN, 2, 3, 2, 8, 2, EPI_GLU>(a, s);
+  if (tiles(m, 16) == 3 && tiles(2 * units, CUS) == 2 * tiles(units, CUS))
+    return launch_one<SIX, PLAIN, 2, 3, 2, 8, 2, EPI_GLU>(a, s);
   return launch_one<SIX, PLAIN, 2, 2, 2, 8, 2, EPI_GLU>(a, s);
 }
 

@@ -49,7 +49,7 @@ def test_where_the_gemv_ends(m):
 
 @pytest.mark.parametrize("relaxed", [1, 0])
 @pytest.mark.parametrize("six", [0, 1])
-@pytest.mark.parametrize("hidden,m", [(96, 5), (2784, 16), (2784, 40), (2784, 97)])
+@pytest.mark.parametrize("hidden,m", [(96, 5), (2784, 16), (2784, 40), (4160, 40), (2784, 97)])
 def test_swiglu_epilogue_bits(hidden, m, six, relaxed):
     """a prompt block whose w1 / w3 GEMM finishes the SwiGLU: the second layer's keys and values follow from every token's
     output of the first layer's"""
