@@ -461,12 +461,27 @@ __global__ __launch_bounds__(256 * RB) __attribute__((amdgpu_waves_per_eu(2))) v
   }
 }
 
+int64_t tiles(int64_t n, int64_t size) { return (n + size - 1) / size; }
+
 template <bool SIX, bool PLAIN, int RT, int TT, int RB, int CK, int D, int EPI>
 hipError_t launch_one(const MatArgs &a, hipStream_t s) {
   using P = Chains<SIX, PLAIN, RT, TT, RB, CK, D, EPI>;
-  const int rows = a.total_rows;
-  const int64_t blocks = (int64_t)((rows + P::ROWS - 1) / P::ROWS) * ((a.m + P::TOKENS - 1) / P::TOKENS);
-  if (blocks > (1ll << 30)) return hipErrorInvalidValue;
+  const int64_t row_blocks = tiles(a.total_rows, P::ROWS), token_blocks = tiles(a.m, P::TOKENS), blocks = row_blocks * token_blocks;
+  // a launch has fewer than 2^32 threads (more are dropped without an error): the tokens in pieces
+  const int64_t most = (int64_t)(UINT32_MAX / P::NT) / row_blocks;
+  if (token_blocks > most) {
+    if (most < 1 || EPI != EPI_STORE || a.qkv.on) return hipErrorInvalidValue;
+    for (int64_t t0 = 0; t0 < a.m; t0 += most * P::TOKENS) {
+      MatArgs p = a;
+      p.m = (int32_t)std::min<int64_t>(most * P::TOKENS, a.m - t0);
+      p.xq = a.xq + t0 * a.xq_stride;
+      p.xs = a.xs + t0 * a.xs_stride;
+      for (int i = 0; i < a.nseg; ++i) p.seg[i].y = a.seg[i].y + t0 * a.seg[i].y_stride;
+      const hipError_t e = launch_one<SIX, PLAIN, RT, TT, RB, CK, D, EPI>(p, s);
+      if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
+  }
   if (P::LDS > 64 * 1024) {
     static bool sized = false;  // once a process: let the kernel take LDS past 64 KiB
     if (!sized) {
@@ -488,7 +503,6 @@ hipError_t launch_one(const MatArgs &a, hipStream_t s) {
 //     for 64 x 32; two a CU, 4096 x 4096, 100 tokens: 19.1 against 16.3);
 //   64 x 32, 8 waves: the rest (a token's operand read once for four row tiles of the block).
 constexpr int CUS = 256;
-int64_t tiles(int64_t n, int64_t size) { return (n + size - 1) / size; }
 
 template <bool SIX, bool PLAIN>
 hipError_t launch_tile(const MatArgs &a, hipStream_t s) {
@@ -534,7 +548,9 @@ hipError_t launch_gelu_tile(const MatArgs &a, hipStream_t s) {
 // rows, 100 tokens (one of theirs a CU, 896 of these) 9.3 / 11.0, 4096 rows, 256 tokens (512) 8.8 / 7.3; K of 192, 14336 rows,
 // 100 tokens 11.5 / 12.0, 6144 rows, 400 tokens (1248 in a round) 16.2 / 14.0; K of 320, 28672 rows, 400 tokens (1456 a round)
 // 54.8 / 58.3, 6144 rows, 400 tokens 18.2 / 16.4; K of 512, 28672 rows, 400 tokens 64.4 / 59.1.
+// (Past 2^27 rows the tile of 16 x 16 would have more threads than a launch takes: theirs.)
 bool gemm_chains_faster(int32_t rows, int32_t m, int32_t k, bool glu) {
+  if (rows > 1 << 27) return false;
   const int64_t theirs = tiles(rows, 64) * tiles(m, 128), ours = tiles(rows, 64) * tiles(m, 32);
   const int64_t rounds = tiles(theirs, 2 * CUS);
   if (glu) return ours <= (theirs <= CUS ? 720 : 1000 * rounds);

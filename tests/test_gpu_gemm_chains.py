@@ -1,6 +1,8 @@
 """The matmuls of more tokens than the GEMV takes, to the bit of the oracle, at the edges of the GEMM's tiles and of the
 rules that pick one: 16 x 16, 32 x 32 and 64 x 32 blocks with a lane chain a wave, the 64 x 128 blocks of full grids, and
 the SwiGLU epilogue's 16, 32 and 48 tokens; both biases, int8 and int6, every number of groups past the fours."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -127,3 +129,23 @@ def test_short_rows_finish_qkv():
     assert same_bits(kv["keys"], k.reshape(-1)) and same_bits(kv["values"], v.reshape(-1))
     eng.release()
     ref.close()
+
+
+def test_more_outputs_than_a_launch_has_threads():
+    """bias 0, 131,072 rows x 131,136 tokens (69 GB of results): four outputs a thread are more than 2^32 threads"""
+    rows, m, k = 1 << 17, (1 << 17) + 64, 32
+    w, ws = weights(rows, k, 0)
+    xq, xs = activations(m, k, 0)
+    y = ctypes.c_void_p()
+    gl.hip_check(gl.hip().hipMalloc(ctypes.byref(y), 4 * rows * m))
+    try:
+        args = [gl.upload(a) for a in (xq, np.ascontiguousarray(xs, np.float32), w, np.ascontiguousarray(ws, np.float32))]
+        gl.check(package().library().hk_matmul(y, *(a.ptr for a in args), m, rows, k, 0, 0, None))
+        gl.hip_check(gl.hip().hipDeviceSynchronize())
+        row = np.zeros(rows, np.float32)
+        for t in (0, 63, 70000, (1 << 17) - 1, 1 << 17, m - 1):
+            gl.hip_check(gl.hip().hipMemcpy(ctypes.c_void_p(row.ctypes.data), ctypes.c_void_p(y.value + 4 * rows * t), row.nbytes, 2))
+            assert same_bits(row, ol.matmul(xq[t:t + 1], xs[t:t + 1], w, ws, rows, k, 0, 0)[0]), t
+    finally:
+        gl.hip().hipDeviceSynchronize()
+        gl.hip().hipFree(y)
