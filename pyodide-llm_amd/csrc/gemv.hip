@@ -994,19 +994,29 @@ int32_t gemv_tokens(int32_t k, bool relaxed) {
 }
 
 // The GEMM's block for a few tokens takes 16 rows through K stage by stage, which no other block of the CU hides: up to
-// 4096 rows 2.6 us and 1.05 ns a value of K (int6 1.2, bias 0 3.2), whatever the rows. The GEMV's time goes with the tokens
-// and with its blocks of four rows a CU (q), and falls only slightly with K, so it is the faster one for few rows, few
-// tokens and long rows. Measured, us a launch (each launch its own weights) here / in the GEMM:
+// 4096 rows 2.6 us and 1.05 ns a value of K (int6 1.2, bias 0 3.2), whatever the rows; bias 0 goes up in steps of 4096 rows (a
+// second, third block a CU: 3.9, 5.3). The GEMV's time goes with the tokens and with its blocks of four rows a CU (q), and
+// falls only slightly with K, so it is the faster one for few rows, few tokens and long rows. Measured, us a launch (each
+// launch its own weights) here / in the GEMM:
 //   bias 64, int8: 1024 rows of 4096, 2 tokens 4.9 / 7.4, 7 tokens 6.7 / 7.5; of 512, 4 tokens 3.4 / 3.3; 512 rows of 14336,
 //     7 tokens 15.8 / 17.7, 8 tokens 19.0 / 17.7; 2048 rows of 4096, 6 tokens 7.1 / 7.6, 8 tokens 8.2 / 7.5; of 1024, 4 tokens
-//     4.8 / 4.4; of 14336, 5 tokens 17.3 / 18.3, 6 tokens 19.4 / 18.3; 3072 rows of 4096, 4 tokens slower, of 8192, 2 tokens
-//     faster; 4096 rows of 4096, 2 tokens 10.7 / 8.4;
+//     4.8 / 4.4; of 14336, 5 tokens 17.3 / 18.3, 6 tokens 19.4 / 18.3; 3072 rows of 4096, 3 tokens 7.0 / 7.8, 4 tokens 7.9 / 7.8
+//     (2 tokens, which request more at once, 8.6 / 7.8), of 8192, 2 tokens 11.0 / 11.9; 4096 rows of 4096, 2 tokens 10.7 / 8.4, of
+//     1024, 5 tokens 5.3 / 5.9, 4 tokens 6.8 / 5.9;
 //   bias 64, int6 (fewer bytes a row): 1024 rows of 14336, 2 tokens 8.5 / 19.9, 8 tokens 16.3 / 20.0; of 512, 4 tokens 3.9 / 3.3;
-//     2048 rows of 4096, 8 tokens 7.2 / 8.1; of 1024, 4 tokens 5.9 / 4.7; 4096 rows of 14336, 2 tokens 18.1 / 20.3, 3 tokens
-//     21.7 / 20.3;
+//     of 28672 in two passes, 5 tokens 25.0 / 35.2, 8 tokens 30.8 / 35.1, of 18944, 7 tokens 23.8 / 24.7, 8 tokens 26.5 / 24.6;
+//     2048 rows of 4096, 8 tokens 7.2 / 8.1; of 1024, 4 tokens 5.9 / 4.7; 3072 rows of 4096, 5 tokens 6.5 / 8.1, 7 tokens 9.3 / 8.2;
+//     of 6144, 5 tokens 11.3 / 10.6, of 12,288, 5 tokens 17.2 / 17.6; 5120 rows of 16384, 2 tokens 23.4 / 27.0, of 18944 34.1 /
+//     30.2; 4096 rows of 14336, 2 tokens 18.1 / 20.3, 3 tokens 21.7 / 20.3;
 //   bias 0 (four sums a group): 1024 rows of 4096, 7 tokens (one pass) 8.2 / 16.4, int6 6.0 / 16.6; 96 rows of 14336 in
-//     passes of 2, 7 tokens 44.4 / 48.1; 1536 rows of 6144, 10 tokens (two passes) int6 16.9 / 23.1; 8192 rows of 4096,
-//     7 tokens 33.5 / 21.0; 1024 rows of 3072, 14 tokens slower, int6 11.2 / 13.3.
+//     passes of 2, 7 tokens 44.4 / 48.1; 1536 rows of 6144, 10 tokens (two passes) int6 16.9 / 23.1; 2048 rows of 9728 in passes
+//     of 3, 7 tokens 31.0 / 33.9, 9 tokens 34.4 / 33.9; of 15360, int6, 8 tokens (four passes) 49.4 / 52.1; 1024 rows of 3072, 14
+//     tokens slower, int6 11.2 / 13.3;
+//   bias 0 past 4096 rows: 5120 rows of 4096, 7 tokens (one pass) int6 15.5 / 19.4, int8 22.1 / 20.1, of 3072 15.6 / 16.4; in two
+//     passes 5120 rows of 8192, 4 tokens 31.3 / 35.6, of 9728 45.4 / 41.7 (int6 38.2 / 40.3), of 14336 63.6 / 59.4 (int6 51.7 /
+//     60.7 at 15360), of 15360, 3 tokens 52.2 / 62.5, int6 45.1 / 61.0, of 24576, 2 tokens 65.2 / 98.2; 7168 rows of 15360, 3 tokens
+//     67.1 / 63.5, int6 57.6 / 61.5; 16,384 rows of 16352, 2 tokens 111 / 119, of 18944 138 / 140; 7168 rows of 24576 87.7 / 98.1,
+//     10,240 rows 118.3 / 133.2, 12,288 rows 137.6 / 134.8, of 28672, 6144 rows 100.6 / 113.8, 7168 rows 121.4 / 114.0; 8192 rows of 4096, 7 tokens 33.5 / 21.0.
 bool gemv_faster(int32_t rows, int32_t k, int32_t m, bool six, bool relaxed) {
   if (m == 1) return true;
   const int32_t step = gemv_tokens(k, relaxed), q = (rows - 1) / 1024 + 1;  // four-row blocks a CU of 256
@@ -1017,18 +1027,41 @@ bool gemv_faster(int32_t rows, int32_t k, int32_t m, bool six, bool relaxed) {
       int32_t k, m;  // the shortest rows, the most tokens
     };
     const Line int8[4] = {{600, k > 8192 ? 7 : 8}, {1800, k > 8192 ? 5 : 6}, {7000, 3}, {INT32_MAX, 0}};
-    const Line int6[4] = {{850, 8}, {2048, k > 16384 ? 6 : 8}, {7000, 3}, {12000, 2}};
-    if (q > 4 || passes > 1) return false;
+    const Line int6[4] = {{850, 8}, {2048, k > 16384 ? 6 : 8}, {7000, k > 16384 ? 4 : 5}, {12000, 2}};
+    if (passes > 1) {
+      if (six) return q == 1 && m <= (rows <= 512 || k >= 20 * 1024 ? 8 : 7);
+      return rows <= 512 && k >= 28 * 1024 && m <= (k >= 40 * 1024 ? 6 : 5);
+    }
+    // (launches of 3 tokens and of 5 and 6 request 4 and 2 KiB of a row at once, where those of 2 and 4 request 8 and 4: rows
+    // that are short, or whole requests, waste less)
+    if (q == 3 && m == 3) return k >= (six ? 4096 : 3072);
+    if (q == 3 && six && (m == 5 || m == 6) && k >= 3072 && k <= 4608) return true;
+    if (q == 4 && !six && m == 5 && k <= 1024) return true;
+    if (q == 5) return six ? m == 2 && k >= 12000 && (k <= 16384 || k >= 24 * 1024) : m == 3 && k > 3584 && k <= 4096;
+    if (q > 4) return false;
     const Line line = six ? int6[q - 1] : int8[q - 1];
     return k >= line.k && m <= line.m;
   }
   if (m <= 6 && passes == 1) return true;
+  if (q > 4) {  // (rows of whole requests again; then two passes: K just past what fewer passes take costs least)
+    if (passes == 1 && six) {
+      return k <= 4096 && (m == 7 ? (q == 5 && k >= 2048) || (q == 6 && k >= 3584) : q == 5 && k >= 3584);
+    }
+    if (passes == 1) return m == 7 && q == 5 && k >= 2048 && k <= 3072;
+    if (step == 1 && m == 3) return q == 5 && k < 17000;
+    if (passes > 2) return false;
+    if (step == 1) return k <= 18 * 1024 || q <= (six || k < 26000 ? 10 : 6);
+    if (step == 2 && m == 3) return q <= (six ? 7 : 6) || q == 9 || (six && q == 10);
+    return m == 4 && q == 5 && (step == 2 ? six || k < 14000 : step == 3 && (six || k < 9000));
+  }
   const int32_t most = six ? 16 : 12;
-  if (q > 4) return false;
   if (step == 8) {  // (rows of up to 3.9 KiB)
     return m <= 8 ? k >= (q < 4 ? 320 * q : 2048) : q == 1 && k >= 2048 && m <= most;
   }
-  return m <= most && passes <= std::max(step > 3 ? 1 : 2, (step > 3 ? 4 : (six && step == 3 ? 8 : 7) - step) - q);
+  if (m > most) return false;
+  if (step > 3) return passes <= std::max(1, 4 - q);
+  const bool more = six ? step == 3 || (step == 2 && k >= 15000) || (k >= 24 * 1024 && q < 3) : step == 3 && q == 2 && m <= 8;
+  return passes <= std::max(2, 7 - step - q + (more ? 1 : 0));
 }
 
 bool decode_takes_f32(int32_t k, bool six, bool relaxed) {
