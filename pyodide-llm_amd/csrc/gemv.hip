@@ -244,9 +244,12 @@ __global__ __launch_bounds__(256) void gemv_kernel(const MatArgs a) {
       const float *tl = P + lane * lay.stride + 4 * lay.q;
       for (int g = G4; g < G; ++g) sum = sum + tl[g - G4];
     }
-    float *y = sg.y + (int64_t)lane * sg.y_stride + r;
-    const float o = sg.accumulate ? *y + sum : sum;
-    *y = sg.bias ? o + sg.bias[r] : o;
+    int late = row;  // (the row's place looked up again: kept from above, it is held in registers through the rows' loads)
+    asm volatile("" : "+v"(late));
+    const RowAt at = row_at(a, late);
+    float *y = at.y + (int64_t)lane * at.y_stride + at.r;
+    const float o = at.accumulate ? *y + sum : sum;
+    *y = at.bias ? o + at.bias[at.r] : o;
   }
 }
 
