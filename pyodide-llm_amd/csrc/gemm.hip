@@ -384,9 +384,6 @@ hipError_t launch_gemm(const MatArgs &a, bool six, bool relaxed, hipStream_t s) 
   return hipGetLastError();
 }
 
-// (the line of long rows for every K: an epilogue saves a launch)
-bool gemm_finishes(int32_t rows, int32_t m, bool relaxed) { return !relaxed || gemm_chains_faster(rows, m, INT32_MAX, false); }
-
 // a quantized output of `hidden` units: its 4-byte runs and its scales aligned and inside [m][q_stride] / [m][s_stride]
 static bool takes_units(const GluOut &g, int32_t hidden) {
   return hidden >= 32 && hidden % 32 == 0 && g.q && g.s && (g.bias == 0 || g.bias == 64) && g.q_stride >= hidden &&

@@ -536,26 +536,50 @@ hipError_t launch_gelu_tile(const MatArgs &a, hipStream_t s) {
   return launch_one<SIX, PLAIN, 1, 2, 2, 8, 2, EPI_GELU>(a, s);
 }
 
-}  // namespace
-
 // gemm.hip's blocks (64 rows x 128 tokens, two a CU) take a K step of 128 in about 1.85 us while at most one lies on a
 // CU, 2.3 us with two, and 2.2 us a round of 512 after that; here the time goes with the blocks of 64 x 32, 1.48 ns a
 // block and K step (the SwiGLU's: 2.2). Measured on both sides of the line (us here / there): 4096 x 4096, 512 tokens
 // 46.9 / 60.4, 1024 tokens 92.4 / 76.0; 6144 x 4096, 384 tokens 57.0 / 66.5, 512 tokens 69.4 / 67.4; 14336 x 4096, 100
 // tokens 48.5 / 59.9, 200 tokens 78.7 / 72.7, 300 tokens (a second round there) 101.9 / 124.2; the SwiGLU at 28672 x
 // 4096, 64 tokens 57.0 / 65.6, 96 tokens 73.6 / 66.9, at 4096 x 512, 300 tokens 11.3 / 12.1, 511 tokens 14.1 / 12.3.
-// Short rows leave the blocks' hand-over and stores, which weigh more on blocks of 64 x 32 (us there / here): K of 96, 14336
-// rows, 100 tokens (one of theirs a CU, 896 of these) 9.3 / 11.0, 4096 rows, 256 tokens (512) 8.8 / 7.3; K of 192, 14336 rows,
-// 100 tokens 11.5 / 12.0, 6144 rows, 400 tokens (1248 in a round) 16.2 / 14.0; K of 320, 28672 rows, 400 tokens (1456 a round)
-// 54.8 / 58.3, 6144 rows, 400 tokens 18.2 / 16.4; K of 512, 28672 rows, 400 tokens 64.4 / 59.1.
+// So a round of theirs is worth 1420 of these (int8 up to 1500, int6 from 1340), and fewer with groups past the fours, whose
+// products meet in a hand-over of their own, and for short rows, where the hand-over and the stores weigh more on blocks of
+// 64 x 32 (us there / here, [blocks there, here]): 18,944 x 14336, int6, 455 tokens [1184, 4440] 617 / 665; 28,672 x 3104 (97 groups), 83
+// tokens [445, 1335] 57.1 / 64.0; 11,344 x 1056 (33), 505 tokens [712, 2848] 47.2 / 54.2; K of 384, 13,420 rows, 607 tokens [1050,
+// 3990] the fewer here by 1.3; K of 192, 14336 rows, 100 tokens [224, 896] 11.5 / 12.0, 5105 rows, 524 tokens [400, 1360] 16.1 / 18.9,
+// 6144 rows, 400 tokens [384, 1248] 16.2 / 14.0; K of 128, 12,084 rows, 175 tokens [378, 1134] 14.1 / 11.7; K of 96, 4096 rows, 256
+// tokens [128, 512: two a CU] 8.8 / 7.3, 4621 rows, 242 tokens [146, 584] 8.3 / 11.1, 22,042 rows, 65 tokens [345, 1035] 10.0 / 14.5.
+// Over 3200 shapes of up to 32,768 rows, K of 96-17,000 and 1024 tokens the choice costs 0.13% of the faster one's time in the mean,
+// and is the 64 x 128 blocks' by more than 4% of their time for 11.
 // (Past 2^27 rows the tile of 16 x 16 would have more threads than a launch takes: theirs.)
+struct Grids {
+  int64_t theirs, ours, rounds;
+};
+Grids grids(int32_t rows, int32_t m) {
+  const int64_t theirs = tiles(rows, 64) * tiles(m, 128);
+  return {theirs, tiles(rows, 64) * tiles(m, 32), tiles(theirs, 2 * CUS)};
+}
+}  // namespace
+
 bool gemm_chains_faster(int32_t rows, int32_t m, int32_t k, bool glu) {
   if (rows > 1 << 27) return false;
-  const int64_t theirs = tiles(rows, 64) * tiles(m, 128), ours = tiles(rows, 64) * tiles(m, 32);
-  const int64_t rounds = tiles(theirs, 2 * CUS);
-  if (glu) return ours <= (theirs <= CUS ? 720 : 1000 * rounds);
-  if (theirs <= CUS) return ours <= (k < 512 ? std::max(512, std::min(1250, 440 + 2 * k)) : 1250);
-  return ours <= (k < 512 ? 1400 : 1480) * rounds;
+  const Grids g = grids(rows, m);
+  if (glu) return g.ours <= (g.theirs <= CUS ? 720 : 1000 * g.rounds);
+  const bool past = k % 128 != 0;  // groups past the fours
+  if (g.theirs <= CUS) {
+    if (k < 128) return g.ours <= 512;
+    return g.ours <= (past ? (k < 256 ? 520 : (k < 1024 ? 760 : 1250)) : (k < 256 ? 700 : (k < 384 ? 820 : 1250)));
+  }
+  if (k < 128) return g.ours <= 440 * g.rounds;
+  return g.ours <= (past ? (k < 1024 ? 1080 : 1270) : (k <= 512 ? 1340 : 1420)) * g.rounds;
+}
+
+// (an epilogue saves a launch: 1480 a round for every K)
+bool gemm_finishes(int32_t rows, int32_t m, bool relaxed) {
+  if (!relaxed) return true;
+  if (rows > 1 << 27) return false;
+  const Grids g = grids(rows, m);
+  return g.ours <= (g.theirs <= CUS ? 1250 : 1480 * g.rounds);
 }
 
 hipError_t launch_gemm_chains(const MatArgs &a, bool six, bool relaxed, hipStream_t s) {

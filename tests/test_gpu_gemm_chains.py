@@ -30,14 +30,23 @@ def test_matmul_bits(rows, k, m, six, bias):
     assert same_bits(gl.matmul(xq, xs, w, ws, rows, k, bias, six), ol.matmul(xq, xs, w, ws, rows, k, bias, six))
 
 
-# rows shorter than 512 leave the chains' blocks for the 64 x 128 ones earlier: of 96 values 429 blocks stay and 680 do not, of
-# 32 495 stay; past one of those a CU 1469 blocks of 512 values stay, and of 480 do not
+# the last grids (in blocks of 64 x 32) that stay, and the first that leave for the 64 x 128 ones: of 96 values 504 / 525, of 128
+# 700 / 702, of 224 520 / 528, of 256 820 / 828, of 992 756 / 768; past one of those a CU of 96 none, of 128 1340 / 1344, of 160
+# 1080 / 1088, of 640 1420 / 1424, of 1120 1268 / 1272
+STAY = [(2688, 96, 384), (1600, 128, 896), (4160, 224, 256), (2624, 256, 640), (2304, 992, 672), (21440, 128, 100), (17280, 160, 100),
+        (22720, 640, 128), (20288, 1120, 128)]
+LEAVE = [(4800, 96, 224), (2496, 128, 576), (2112, 224, 512), (2944, 256, 576), (2048, 992, 768), (16448, 96, 65), (21504, 128, 128),
+         (17408, 160, 128), (22784, 640, 128), (20352, 1120, 128)]
+
+
 @pytest.mark.parametrize("six", [0, 1])
-@pytest.mark.parametrize("rows,k,m", [(2112, 96, 416), (2176, 96, 640), (2112, 32, 480), (7232, 480, 416), (7232, 512, 416)])
-def test_short_rows(rows, k, m, six):
+@pytest.mark.parametrize("rows,k,m", STAY + LEAVE)
+def test_where_the_64_x_128_blocks_start(rows, k, m, six):
     w, ws = weights(rows, k, six)
     xq, xs = activations(m, k, 64)
-    assert same_bits(gl.matmul(xq, xs, w, ws, rows, k, 64, six), ol.matmul(xq, xs, w, ws, rows, k, 64, six))
+    some = np.r_[0:rows - 64:7, rows - 64:rows]  # (the oracle's rows: every seventh, the last block's all)
+    got = gl.matmul(xq, xs, w, ws, rows, k, 64, six)[:, some]
+    assert same_bits(got, ol.matmul(xq, xs, w[some], ws[some], len(some), k, 64, six))
 
 
 @pytest.mark.parametrize("m", [2, 6, 7, 8, 9])
