@@ -229,6 +229,10 @@ __global__ __launch_bounds__(256) void gemv_kernel(const MatArgs a) {
     }
   }
   if constexpr (SUMS) return;
+  // (of several tokens the row's place looked up again: kept from above, it is held in registers through the rows' loads)
+  int late = row;
+  if constexpr (M > 1) asm volatile("" : "+v"(late));
+  const RowAt at = M > 1 ? row_at(a, late) : sg;
   wave_sync_lds();
   float chain = 0.0f;  // lane 4t + k (t < M): accumulator k of token t
   if (lane < 4 * M) {
@@ -244,9 +248,6 @@ __global__ __launch_bounds__(256) void gemv_kernel(const MatArgs a) {
       const float *tl = P + lane * lay.stride + 4 * lay.q;
       for (int g = G4; g < G; ++g) sum = sum + tl[g - G4];
     }
-    int late = row;  // (the row's place looked up again: kept from above, it is held in registers through the rows' loads)
-    asm volatile("" : "+v"(late));
-    const RowAt at = row_at(a, late);
     float *y = at.y + (int64_t)lane * at.y_stride + at.r;
     const float o = at.accumulate ? *y + sum : sum;
     *y = at.bias ? o + at.bias[at.r] : o;
@@ -1013,7 +1014,7 @@ int32_t gemv_tokens(int32_t k, bool relaxed) {
 //     30.2; 4096 rows of 14336, 2 tokens 18.1 / 20.3, 3 tokens 21.7 / 20.3;
 //   bias 0 (four sums a group): 1024 rows of 4096, 7 tokens (one pass) 8.2 / 16.4, int6 6.0 / 16.6; 96 rows of 14336 in
 //     passes of 2, 7 tokens 44.4 / 48.1; 1536 rows of 6144, 10 tokens (two passes) int6 16.9 / 23.1; 2048 rows of 9728 in passes
-//     of 3, 7 tokens 31.0 / 33.9, 9 tokens 34.4 / 33.9; of 15360, int6, 8 tokens (four passes) 49.4 / 52.1; 1024 rows of 3072, 14
+//     of 3, 7 tokens 31.0 / 33.9, 9 tokens 34.4 / 33.9; of 4096 in two, 9 tokens 16.2 / 16.2, 12 tokens 17.6 / 16.2, int6 14.3 / 16.4; of 15360, int6, 8 tokens (four passes) 49.4 / 52.1; 1024 rows of 3072, 14
 //     tokens slower, int6 11.2 / 13.3;
 //   bias 0 past 4096 rows: 5120 rows of 4096, 7 tokens (one pass) int6 15.5 / 19.4, int8 22.1 / 20.1, of 3072 15.6 / 16.4; in two
 //     passes 5120 rows of 8192, 4 tokens 31.3 / 35.6, of 9728 45.4 / 41.7 (int6 38.2 / 40.3), of 14336 63.6 / 59.4 (int6 51.7 /
@@ -1057,7 +1058,7 @@ bool gemv_faster(int32_t rows, int32_t k, int32_t m, bool six, bool relaxed) {
     if (step == 2 && m == 3) return q <= (six ? 7 : 6) || q == 9 || (six && q == 10);
     return m == 4 && q == 5 && (step == 2 ? six || k < 14000 : step == 3 && (six || k < 9000));
   }
-  const int32_t most = six ? 16 : 12;
+  const int32_t most = six ? 16 : (q == 1 ? 12 : 10);
   if (step == 8) {  // (rows of up to 3.9 KiB)
     return m <= 8 ? k >= (q < 4 ? 320 * q : 2048) : q == 1 && k >= 2048 && m <= most;
   }

@@ -23,7 +23,7 @@ INT6 = [(33, 832, 8), (33, 864, 8), (1025, 2016, 8), (1025, 2048, 8), (1030, 164
         (4100, 12000, 2), (4100, 16416, 2), (33, 18944, 8), (513, 18944, 8), (513, 20480, 8), (1025, 20480, 8)]
 # bias 0: one pass of 8, then of 7, 3, 2 and 1
 PLAIN = [(33, 288, 7), (33, 320, 7), (33, 320, 9), (1025, 640, 8), (33, 2048, 12), (33, 2048, 16), (33, 2048, 17),
-         (1025, 2048, 9), (33, 4096, 9), (1025, 4096, 12), (2050, 4096, 8), (33, 8192, 9), (33, 8192, 12), (1025, 8192, 6),
+         (1025, 2048, 9), (33, 4096, 9), (1025, 4096, 10), (1025, 4096, 12), (2050, 4096, 8), (33, 8192, 9), (33, 8192, 12), (1025, 8192, 6),
          (33, 14336, 8), (33, 14336, 9), (1025, 14336, 6), (33, 18944, 5), (33, 18944, 6), (3073, 18944, 2),
          (1025, 8192, 7), (1025, 8192, 9), (1025, 15360, 8), (33, 24576, 6), (1025, 24576, 5)]
 # and past 4096 rows: one pass of 7 and 8, two of 3, 2 and 1, three of 1
