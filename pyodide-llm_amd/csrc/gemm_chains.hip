@@ -544,9 +544,9 @@ hipError_t launch_gelu_tile(const MatArgs &a, hipStream_t s) {
 // 4096, 64 tokens 57.0 / 65.6, 96 tokens 73.6 / 66.9, at 4096 x 512, 300 tokens 11.3 / 12.1, 511 tokens 14.1 / 12.3.
 // So a round of theirs is worth 1420 of these (int8 up to 1500, int6 from 1340), and fewer with groups past the fours, whose
 // products meet in a hand-over of their own, and for short rows, where the hand-over and the stores weigh more on blocks of
-// 64 x 32 (us there / here, [blocks there, here]): 18,944 x 14336, int6, 455 tokens [1184, 4440] 617 / 665; 28,672 x 3104 (97 groups), 83
+// 64 x 32 (us there / here, [blocks there, here]): 18,944 x 14336, int6, 455 tokens [1184, 4440] 617 / 665; 28,460 x 3104 (97 groups), 83
 // tokens [445, 1335] 57.1 / 64.0; 11,344 x 1056 (33), 505 tokens [712, 2848] 47.2 / 54.2; K of 384, 13,420 rows, 607 tokens [1050,
-// 3990] the fewer here by 1.3; K of 192, 14336 rows, 100 tokens [224, 896] 11.5 / 12.0, 5105 rows, 524 tokens [400, 1360] 16.1 / 18.9,
+// 3990] 46.3 / 35.7; K of 192, 14336 rows, 100 tokens [224, 896] 11.5 / 12.0, 5105 rows, 524 tokens [400, 1360] 16.1 / 18.9,
 // 6144 rows, 400 tokens [384, 1248] 16.2 / 14.0; K of 128, 12,084 rows, 175 tokens [378, 1134] 14.1 / 11.7; K of 96, 4096 rows, 256
 // tokens [128, 512: two a CU] 8.8 / 7.3, 4621 rows, 242 tokens [146, 584] 8.3 / 11.1, 22,042 rows, 65 tokens [345, 1035] 10.0 / 14.5.
 // Over 3200 shapes of up to 32,768 rows, K of 96-17,000 and 1024 tokens the choice costs 0.13% of the faster one's time in the mean,
